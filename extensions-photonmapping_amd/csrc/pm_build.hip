@@ -2548,6 +2548,7 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
         }
     }
     ctx->has_boxes = prm.propagate_aabbs != 0;
+    ctx->wide_leaves = LS > 32;
     if (!graph) {
         ctx->upper_levels = h.level;
         ctx->lower_levels = h.lower_levels;
@@ -2657,6 +2658,7 @@ void reserve_build_caps(pm_ctx *ctx, const BuildSizes &caps, int N, hipStream_t 
     sc.lower_careas.reserve(2 * (size_t)caps.lower, s);
     sc.prims_part.reserve(PRIM_SLOTS, s);
     ctx->packed.reserve((size_t)caps.nodes + 1, s);
+    ctx->leaf_rec.reserve(2 * (size_t)caps.nodes + 2, s);
     reserve_scan_tmp(sc, std::max({2 * caps.active, caps.segs, caps.lower}), s);
     sc.lvl.reserve(1, s);
 }
@@ -2741,7 +2743,7 @@ std::vector<void **> graph_buffers(pm_ctx *ctx) {
         (void **)&a.info.ptr, (void **)&a.split.ptr, (void **)&a.bmin.ptr, (void **)&a.bmax.ptr,
         (void **)&a.prim_index.ptr, (void **)&a.bitmap.ptr, (void **)&a.children.ptr, (void **)&a.area.ptr,
         (void **)&a.parent.ptr, (void **)&ctx->prim_indices.ptr, (void **)&ctx->leaf_ids.ptr,
-        (void **)&ctx->packed.ptr, (void **)&ctx->leaf_tris.ptr, (void **)&sc.prim_min.ptr,
+        (void **)&ctx->packed.ptr, (void **)&ctx->leaf_rec.ptr, (void **)&ctx->leaf_tris.ptr, (void **)&sc.prim_min.ptr,
         (void **)&sc.prim_max.ptr, (void **)&sc.segL.ptr, (void **)&sc.segR.ptr,
         (void **)&sc.segLoff.ptr, (void **)&sc.segRoff.ptr, (void **)&sc.node_lna.ptr, (void **)&sc.node_lref.ptr,
         (void **)&sc.node_lseg.ptr, (void **)&sc.node_sz.ptr, (void **)&sc.lb_ctr.ptr, (void **)&sc.prims_part.ptr, (void **)&sc.areas.ptr, (void **)&sc.lower_flag.ptr,
@@ -2809,6 +2811,7 @@ void capture_batch(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4
     ctx->graph_p0 = P0; ctx->graph_p1 = P1; ctx->graph_p2 = P2;
     ctx->graph_n = N; ctx->graph_M = M;
     ctx->graph_boxes = bp.propagate_aabbs != 0;
+    ctx->graph_wide = bp.lower_size > 32;
     ctx->graph_offsets = ctx->mesh_offsets;
 
     // 3. record build + trace on the context's own stream (recording runs nothing)
@@ -2866,6 +2869,7 @@ void launch_batch(pm_ctx *ctx, hipStream_t s) {
     ctx->num_roots = ctx->graph_M;
     ctx->mesh_offsets = ctx->graph_offsets;
     ctx->has_boxes = ctx->graph_boxes;
+    ctx->wide_leaves = ctx->graph_wide;
     ctx->has_tree = true;
 }
 

@@ -91,14 +91,10 @@ struct NodeArrays {
 
 // Device view used by the tracers.
 struct TreeDev {
-    const int8_t *info;
-    const float *split;
-    const int2 *children;
-    const int *prim_index;
-    const long long *bitmap;
-    const float4 *bmin, *bmax;
     const int *prim_indices;
     const int4 *packed;        // one 16-byte record per node (trace view)
+    const float4 *leaf_rec;    // 2 float4 per node, leaves only: box min | first slot, box max | bitmap's low word
+    bool wide;                 // bitmaps may reach past bit 31 (the high word: packed)
     const float4 *leaf_tris;   // 3 float4 per leaf slot: v0 (w = id bits), e1, e2
     const float4 *leaf_woop;   // Woop intersection: 3 float4 per leaf slot (m0, m1, m2)
     int num_nodes;
@@ -249,6 +245,8 @@ struct pm_ctx {
     pmkd::DevBuf<int> prim_indices;
     pmkd::DevBuf<int> leaf_ids;
     pmkd::DevBuf<int4> packed;      // trace view: packed nodes
+    pmkd::DevBuf<float4> leaf_rec;  // trace view: the leaves' boxes, first slots and bitmaps
+    bool wide_leaves = false;       // a leaf may hold more than 32 slots
     pmkd::DevBuf<float4> leaf_tris; // trace view: leaf-ordered triangles
     pmkd::DevBuf<float4> woop;      // Woop matrices (per leaf slot or per triangle), per call
     pmkd::BuildScratch scratch;
@@ -267,7 +265,7 @@ struct pm_ctx {
     pmkd::DevBuf<int> graph_off;       // the captured batch's mesh offsets (its own copy)
     const float4 *graph_p0 = nullptr, *graph_p1 = nullptr, *graph_p2 = nullptr;
     int graph_n = 0, graph_M = 0;
-    bool graph_boxes = false;
+    bool graph_boxes = false, graph_wide = false;
     std::vector<int> graph_offsets;
     bool graph_pending = false;        // a replay ran; host-side tree sizes not read back yet
     int num_cus = 0;                   // compute units of the device (0 = not queried yet)
