@@ -372,7 +372,7 @@ __global__ __launch_bounds__(TB) void trace_kernel(TreeDev T, const float4 *__re
     }
 }
 
-// ---- cooperative leaf test (Moller-Trumbore tracers)
+// ---- cooperative leaf test (Moller-Trumbore, and Woop on the slots' matrices)
 //
 // After a wave's lanes have descended to their leaves, lane i holds a leaf
 // with k_i triangles; tested lane by lane the wave would loop max k_i times
@@ -438,10 +438,20 @@ __device__ __forceinline__ void wave_sync() {
 // acceptance, written as min(hx, hy, hz) >= 0, hx <= th, hy + hz <= 1 (fminf
 // returns the other operand of a NaN; a NaN hx fails hx <= th, a NaN hy or
 // hz fails hy + hz <= 1).
+// WOOP: the slot's record is its matrix m0, m1, m2 and the test woop_test's
+// (the lane-per-ray loop waited for each lane's own matrices, one triangle
+// after another: 100,003 probe rays over a 20,011-triangle soup 505 -> 186 us).
+template <bool WOOP>
 __device__ __forceinline__ void coop_pair(const float4 *__restrict__ L, unsigned long long *key, unsigned off,
                                           f3 ro, f3 rd, float rth) {
     const float4 *R3 = reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(L) + off);
     const float4 a0 = R3[0], a1 = R3[1], a2 = R3[2];
+    if constexpr (WOOP) {
+        float t = rth, u, v;
+        if (woop_test(a0, a1, a2, ro, rd, t, u, v))
+            atomicMin(key, ((unsigned long long)__float_as_uint(t + 0.0f) << 32) | (unsigned)~off);
+        return;
+    }
     const f3 v0 = mk3(a0), e1 = mk3(a1), e2 = mk3(a2);
     const f3 p = cross3(rd, e2);
     const f3 t = sub3(ro, v0);
@@ -457,7 +467,7 @@ __device__ __forceinline__ void coop_pair(const float4 *__restrict__ L, unsigned
 // every lane of the wave calls it with the byte offset of its leaf's first
 // record (3 float4 per slot; every offset fits 32 bits); returns the byte
 // offset of the lane's winning record, or -1
-template <bool RECS>
+template <bool RECS, bool WOOP>
 __device__ __forceinline__ long long coop_leaf(const float4 *__restrict__ L, CoopLds<RECS> &C,
                                                unsigned long long bm, unsigned base48, f3 o, f3 d, float th) {
     const int lane = threadIdx.x & 63;
@@ -543,7 +553,7 @@ __device__ __forceinline__ long long coop_leaf(const float4 *__restrict__ L, Coo
             unsigned off;
             int ow4;
             pair_at(r + lane, ro, rd, rth, off, ow4);
-            coop_pair(L, &C.key[ow4 >> 2], off, ro, rd, rth);
+            coop_pair<WOOP>(L, &C.key[ow4 >> 2], off, ro, rd, rth);
         }
         if (r < wn) {
             f3 ro, rd;
@@ -551,7 +561,7 @@ __device__ __forceinline__ long long coop_leaf(const float4 *__restrict__ L, Coo
             unsigned off;
             int ow4;
             pair_at(r + lane, ro, rd, rth, off, ow4);
-            if (r + lane < wn) coop_pair(L, &C.key[ow4 >> 2], off, ro, rd, rth);
+            if (r + lane < wn) coop_pair<WOOP>(L, &C.key[ow4 >> 2], off, ro, rd, rth);
         }
     }
     wave_sync();
@@ -567,7 +577,7 @@ __device__ __forceinline__ long long coop_leaf(const float4 *__restrict__ L, Coo
 // CAPPED: a lane's descent walks at most `cap` inner nodes per iteration and
 // goes on in the next (pm_trace_params.step_cap); the nodes visited, and so
 // records and counters, are the same.
-template <int SMAX, bool SHORT, bool SKIP, bool COUNT, bool CAPPED>
+template <int SMAX, bool SHORT, bool SKIP, bool COUNT, bool CAPPED, bool WOOP>
 __global__ __launch_bounds__(TB) void trace_coop_kernel(TreeDev T, const float4 *__restrict__ org,
                                                         const float4 *__restrict__ dir,
                                                         const int *__restrict__ ray_root,
@@ -679,15 +689,21 @@ __global__ __launch_bounds__(TB) void trace_coop_kernel(TreeDev T, const float4 
             }
         }
         // the leaves, by the whole wave
-        const long long win = coop_leaf(T.leaf_tris, C, bm, (unsigned)base * 48u, R.o, R.d, R.th);
+        const float4 *const recs = WOOP ? T.leaf_woop : T.leaf_tris;
+        const long long win = coop_leaf<!SHORT, WOOP>(recs, C, bm, (unsigned)base * 48u, R.o, R.d, R.th);
         if (q >= 0 && at_leaf) {
             int hit = -1;
             if (win >= 0) {             // the owner's own test of its winner
-                const float4 *W = reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(T.leaf_tris) +
+                const float4 *W = reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(recs) +
                                                                    (unsigned)win);
                 const float4 a0 = W[0];
-                if (mt_edges(mk3(a0), mk3(W[1]), mk3(W[2]), R.o, R.d, R.th, R.tu, R.tv))
-                    hit = __float_as_int(a0.w);
+                if constexpr (WOOP) {
+                    if (woop_test(a0, W[1], W[2], R.o, R.d, R.th, R.tu, R.tv))
+                        hit = T.prim_indices[(unsigned)win / 48u];
+                } else {
+                    if (mt_edges(mk3(a0), mk3(W[1]), mk3(W[2]), R.o, R.d, R.th, R.tu, R.tv))
+                        hit = __float_as_int(a0.w);
+                }
             }
             done = hit != -1 || !(R.th < F_INF);
             if (done) {
@@ -1027,12 +1043,12 @@ void launch_coop(K k, const TreeDev &T, const RayBatch &R, int S, pm_hit *out, i
 template <int SMAX, bool SHORT, bool SKIP, bool COUNT, bool WOOP>
 void launch_trace(const TreeDev &T, const RayBatch &R, int S, pm_hit *out, int4 *cnt, const Launch &L,
                   hipStream_t s) {
-    if (!WOOP && 48ll * T.num_slots < (1ll << 32)) {
+    if (48ll * T.num_slots < (1ll << 32)) {
         if (L.step_cap > 0) {
-            auto k = trace_coop_kernel<SMAX, SHORT, SKIP, COUNT, true>;
+            auto k = trace_coop_kernel<SMAX, SHORT, SKIP, COUNT, true, WOOP>;
             launch_coop(k, T, R, S, out, cnt, L, L.step_cap, s);
         } else {
-            auto k = trace_coop_kernel<SMAX, SHORT, SKIP, COUNT, false>;
+            auto k = trace_coop_kernel<SMAX, SHORT, SKIP, COUNT, false, WOOP>;
             launch_coop(k, T, R, S, out, cnt, L, 0, s);
         }
     } else {
