@@ -569,6 +569,82 @@ __device__ __forceinline__ long long coop_leaf(const float4 *__restrict__ L, Coo
     return best == ~0ull ? -1ll : (long long)(unsigned)~(unsigned)(best & 0xffffffffu);
 }
 
+// ---- canvas shading: ColorKernels.h:15-85 in the tracers' shading loops
+// (Raytracer.cu:165-262, ShortStack.cu:96-194, BruteTracer.cu:54-96); the
+// specular power is the correctly rounded float of the double power
+struct Light { f3 pos, ambient, diffuse, specular; };
+
+__device__ __forceinline__ f3 scale3(f3 a, float s) { return {a.x * s, a.y * s, a.z * s}; }
+__device__ __forceinline__ f3 add3(f3 a, f3 b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
+__device__ __forceinline__ f3 mul3(f3 a, f3 b) { return {a.x * b.x, a.y * b.y, a.z * b.z}; }
+__device__ __forceinline__ float saturate(float x) { return x > 1.0f ? 1.0f : (x > 0.0f ? x : 0.0f); }
+__device__ __forceinline__ float clamp01(float x) { return fmaxf(0.0f, fminf(x, 1.0f)); }
+
+// PhongLighting, ColorKernels.h:15-45, shadow = 1 (the reference's shadow
+// rays are disabled, Raytracer.cu:219-226)
+__device__ __forceinline__ float4 phong(const float4 c, f3 normal, f3 point, f3 origin, const Light &L) {
+    const f3 lightDir = normalize3(sub3(L.pos, point));
+    const float diffuse = saturate(dot3(lightDir, normal) * 1.0f);
+    f3 refl = sub3(scale3(normal, 2.0f * dot3(normal, lightDir)), lightDir);
+    refl = normalize3(refl);
+    const float stemp = saturate(dot3(normalize3(sub3(origin, point)), refl));
+    const float specProp = 1.0f - c.w;
+    const float specular = specProp * (float)pow((double)stemp, (double)(128.0f * specProp));
+    const f3 base = {c.x, c.y, c.z};
+    const f3 light = add3(mul3(base, add3(L.ambient, scale3(L.diffuse, diffuse))),
+                          scale3(scale3(scale3(L.specular, specular), 10.0f), 1.0f));
+    const float alpha = c.w < specular ? specular : c.w;
+    return make_float4(clamp01(light.x), clamp01(light.y), clamp01(light.z), alpha);
+}
+
+// Lighting, ColorKernels.h:47-77: shade the hit, turn the ray into its
+// mirror reflection from the hit point
+__device__ __forceinline__ float4 lighting(const pm_hit &h, f3 &origin, f3 &dir, const float4 *__restrict__ n0,
+                                           const float4 *__restrict__ n1, const float4 *__restrict__ n2,
+                                           const uchar4 *__restrict__ c0, const Light &L) {
+    const f3 point = add3(origin, scale3(dir, h.t));
+    const float w = 1.0f - h.u - h.v;
+    f3 normal = add3(add3(scale3(mk3(n0[h.id]), w), scale3(mk3(n1[h.id]), h.u)), scale3(mk3(n2[h.id]), h.v));
+    normal = normalize3(normal);
+    const uchar4 cc = c0[h.id];
+    const float4 col = make_float4(cc.x / 255.0f, cc.y / 255.0f, cc.z / 255.0f, cc.w / 255.0f);
+    dir = add3(scale3(normal, 2.0f * dot3(normal, scale3(dir, -1.0f))), dir);
+    dir = normalize3(dir);
+    const float4 out = phong(col, normal, point, origin, L);
+    origin = add3(point, scale3(dir, 0.00001f));
+    return out;
+}
+
+// BlendColor, ColorKernels.h:79-84
+__device__ __forceinline__ float4 blend(const float4 o, float4 n) {
+    const float a = n.w;
+    n.w = 1.0f;
+    const float k = (1.0f - o.w) * a;
+    return make_float4(o.x + k * n.x, o.y + k * n.y, o.z + k * n.z, o.w + k * n.w);
+}
+
+// What the cooperative kernel needs to turn first hits into a canvas (CANVAS):
+// a lane keeps its pixel over all bounces, so the mirror rays of some lanes are
+// traced in the same rounds as the first rays of others.  Against the
+// lane-per-ray loop (a lane's leaf triangles one after another, most lanes
+// idle), 1280 x 720 in a 5,316-triangle room: 605 -> 359 us.  The launch has no
+// ray counter: canvas calls on one context share no memory of it, and handing a
+// block's rays out to its waves as lanes fall idle measured slower (542 us with
+// runs of 450 rays, 370 with 256: neighbouring pixels are of like cost, and a
+// refilled lane falls out of step with them).
+struct CanvasArgs {
+    const float4 *n0, *n1, *n2;
+    const uchar4 *c0;
+    Light light;
+    int max_bounces;
+    uchar4 *canvas;
+};
+
+__device__ __forceinline__ uchar4 canvas_pixel(const float4 col) {
+    return make_uchar4((unsigned char)(col.x * 255.0f), (unsigned char)(col.y * 255.0f),
+                       (unsigned char)(col.z * 255.0f), (unsigned char)(col.w * 255.0f));
+}
+
 // the persistent kernel of trace_kernel with the leaf test done by the wave.
 // Lanes below `width` take rays (launch_coop's rule); a wave's first chunk is
 // the one its index names, so that a launch's thousands of waves do not start
@@ -577,14 +653,14 @@ __device__ __forceinline__ long long coop_leaf(const float4 *__restrict__ L, Coo
 // CAPPED: a lane's descent walks at most `cap` inner nodes per iteration and
 // goes on in the next (pm_trace_params.step_cap); the nodes visited, and so
 // records and counters, are the same.
-template <int SMAX, bool SHORT, bool SKIP, bool COUNT, bool CAPPED, bool WOOP>
+template <int SMAX, bool SHORT, bool SKIP, bool COUNT, bool CAPPED, bool WOOP, bool CANVAS = false>
 __global__ __launch_bounds__(TB) void trace_coop_kernel(TreeDev T, const float4 *__restrict__ org,
                                                         const float4 *__restrict__ dir,
                                                         const int *__restrict__ ray_root,
                                                         const unsigned *__restrict__ order, int n, int S,
                                                         pm_hit *__restrict__ out,
                                                         int4 *__restrict__ counters, int *__restrict__ work,
-                                                        int cap, int width) {
+                                                        int cap, int width, CanvasArgs V) {
     __shared__ int stk_rows[2 * (SHORT ? SMAX : 1)][TB];   // short stack: node rows, then tNext rows
     int *const stk = &stk_rows[0][threadIdx.x];
     __shared__ CoopLds<!SHORT> coop[TB / 64];
@@ -605,6 +681,8 @@ __global__ __launch_bounds__(TB) void trace_coop_kernel(TreeDev T, const float4 
     RayState R;
     R.o = {0.0f, 0.0f, 0.0f}; R.d = R.o; R.th = 0.0f;
     int4 cnt = make_int4(0, 0, 0, 0);
+    float4 col = make_float4(0.0f, 0.0f, 0.0f, 0.0f);   // CANVAS: the ray's colour and bounces so far
+    int bounce = 0;
     for (;;) {
         const unsigned long long idle = __ballot(taker && q < 0);
         if (__popcll(idle) >= refill && !exhausted) {
@@ -636,8 +714,13 @@ __global__ __launch_bounds__(TB) void trace_coop_kernel(TreeDev T, const float4 
                     } else if (ray_root_valid(T, ray_root, q, root_id)) {
                         R = ray_start(T, root_id, mk3(org[q]), adjust_dir(mk3(dir[q])));
                         cnt = make_int4(0, 0, 0, 0);
+                        if (CANVAS) {
+                            col = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                            bounce = 0;
+                        }
                     } else {
-                        out[q] = miss_record();
+                        if (CANVAS) V.canvas[q] = make_uchar4(0, 0, 0, 0);
+                        else out[q] = miss_record();
                         if (COUNT) counters[q] = make_int4(0, 0, 0, 0);
                         q = -1;
                     }
@@ -706,13 +789,22 @@ __global__ __launch_bounds__(TB) void trace_coop_kernel(TreeDev T, const float4 
                 }
             }
             done = hit != -1 || !(R.th < F_INF);
+            if (CANVAS && hit != -1) {
+                // shade the hit; the mirror ray goes on in this lane
+                f3 o = R.o, d = R.d;
+                col = blend(col, lighting(ray_record(R, hit), o, d, V.n0, V.n1, V.n2, V.c0, V.light));
+                done = !(col.w < 0.97f) || ++bounce >= V.max_bounces;
+                R = ray_start(T, R.root_id, o, adjust_dir(d));
+            }
             if (done) {
-                out[q] = ray_record(R, hit);
+                if (CANVAS) V.canvas[q] = canvas_pixel(col);
+                else out[q] = ray_record(R, hit);
                 if (COUNT) counters[q] = cnt;
                 q = -1;
             }
         } else if (q >= 0 && done) {    // done before a leaf: a miss
-            out[q] = miss_record();
+            if (CANVAS) V.canvas[q] = canvas_pixel(col);
+            else out[q] = miss_record();
             if (COUNT) counters[q] = cnt;
             q = -1;
         }
@@ -847,60 +939,6 @@ __global__ __launch_bounds__(TB) void leaf_copy_kernel(const int *__restrict__ p
     }
 }
 
-// ---- canvas shading: ColorKernels.h:15-85 in the tracers' shading loops
-// (Raytracer.cu:165-262, ShortStack.cu:96-194, BruteTracer.cu:54-96); the
-// specular power is the correctly rounded float of the double power
-struct Light { f3 pos, ambient, diffuse, specular; };
-
-__device__ __forceinline__ f3 scale3(f3 a, float s) { return {a.x * s, a.y * s, a.z * s}; }
-__device__ __forceinline__ f3 add3(f3 a, f3 b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
-__device__ __forceinline__ f3 mul3(f3 a, f3 b) { return {a.x * b.x, a.y * b.y, a.z * b.z}; }
-__device__ __forceinline__ float saturate(float x) { return x > 1.0f ? 1.0f : (x > 0.0f ? x : 0.0f); }
-__device__ __forceinline__ float clamp01(float x) { return fmaxf(0.0f, fminf(x, 1.0f)); }
-
-// PhongLighting, ColorKernels.h:15-45, shadow = 1 (the reference's shadow
-// rays are disabled, Raytracer.cu:219-226)
-__device__ __forceinline__ float4 phong(const float4 c, f3 normal, f3 point, f3 origin, const Light &L) {
-    const f3 lightDir = normalize3(sub3(L.pos, point));
-    const float diffuse = saturate(dot3(lightDir, normal) * 1.0f);
-    f3 refl = sub3(scale3(normal, 2.0f * dot3(normal, lightDir)), lightDir);
-    refl = normalize3(refl);
-    const float stemp = saturate(dot3(normalize3(sub3(origin, point)), refl));
-    const float specProp = 1.0f - c.w;
-    const float specular = specProp * (float)pow((double)stemp, (double)(128.0f * specProp));
-    const f3 base = {c.x, c.y, c.z};
-    const f3 light = add3(mul3(base, add3(L.ambient, scale3(L.diffuse, diffuse))),
-                          scale3(scale3(scale3(L.specular, specular), 10.0f), 1.0f));
-    const float alpha = c.w < specular ? specular : c.w;
-    return make_float4(clamp01(light.x), clamp01(light.y), clamp01(light.z), alpha);
-}
-
-// Lighting, ColorKernels.h:47-77: shade the hit, turn the ray into its
-// mirror reflection from the hit point
-__device__ __forceinline__ float4 lighting(const pm_hit &h, f3 &origin, f3 &dir, const float4 *__restrict__ n0,
-                                           const float4 *__restrict__ n1, const float4 *__restrict__ n2,
-                                           const uchar4 *__restrict__ c0, const Light &L) {
-    const f3 point = add3(origin, scale3(dir, h.t));
-    const float w = 1.0f - h.u - h.v;
-    f3 normal = add3(add3(scale3(mk3(n0[h.id]), w), scale3(mk3(n1[h.id]), h.u)), scale3(mk3(n2[h.id]), h.v));
-    normal = normalize3(normal);
-    const uchar4 cc = c0[h.id];
-    const float4 col = make_float4(cc.x / 255.0f, cc.y / 255.0f, cc.z / 255.0f, cc.w / 255.0f);
-    dir = add3(scale3(normal, 2.0f * dot3(normal, scale3(dir, -1.0f))), dir);
-    dir = normalize3(dir);
-    const float4 out = phong(col, normal, point, origin, L);
-    origin = add3(point, scale3(dir, 0.00001f));
-    return out;
-}
-
-// BlendColor, ColorKernels.h:79-84
-__device__ __forceinline__ float4 blend(const float4 o, float4 n) {
-    const float a = n.w;
-    n.w = 1.0f;
-    const float k = (1.0f - o.w) * a;
-    return make_float4(o.x + k * n.x, o.y + k * n.y, o.z + k * n.z, o.w + k * n.w);
-}
-
 // brute-force first hit for one ray (Exhaustive, BruteTracer.cu:54-96),
 // straight from global memory
 template <bool WOOP>
@@ -954,8 +992,7 @@ __global__ __launch_bounds__(TB) void canvas_kernel(TreeDev T, const float4 *__r
         if (ALGO != PM_TRACE_BRUTE) d = adjust_dir(d);
         if (!(col.w < 0.97f)) break;
     }
-    canvas[r] = make_uchar4((unsigned char)(col.x * 255.0f), (unsigned char)(col.y * 255.0f),
-                            (unsigned char)(col.z * 255.0f), (unsigned char)(col.w * 255.0f));
+    canvas[r] = canvas_pixel(col);
 }
 
 // CreateWoopValues (GeometryList.cu:80-101): matrices of (p1, p2, p0) for
@@ -1025,19 +1062,20 @@ void clear_work(int *work, hipStream_t s) {
 // with 32, 130 with 64; 1,000 probe rays in a 50,000-triangle soup 80 us with
 // 1 and 228 with 64; past the line (30,000 probes: 143 us with 8 rays a wave,
 // 190 with 4) the extra waves queue.  When every wave's first chunk covers
-// all rays the counter is neither cleared nor read.
+// all rays the counter is neither cleared nor read; a launch without a counter
+// always does that, its later blocks starting as earlier ones end.
 template <class K>
 void launch_coop(K k, const TreeDev &T, const RayBatch &R, int S, pm_hit *out, int4 *cnt, const Launch &L, int cap,
-                 hipStream_t s) {
+                 hipStream_t s, const CanvasArgs &V = CanvasArgs{}) {
     const long long resident = resident_blocks(k, L);
     constexpr int WAVES = TB / 64;
     int width = 64;
     while (width > 1 && R.n <= resident * WAVES * (width / 2)) width /= 2;
     const long long blocks = ((long long)R.n + WAVES * width - 1) / (WAVES * width);
-    const bool one_chunk = blocks <= resident;
+    const bool one_chunk = !L.work || blocks <= resident;
     if (!one_chunk) clear_work(L.work, s);
-    k<<<(int)std::min(blocks, resident), TB, 0, s>>>(T, R.org, R.dir, R.root, R.order, R.n, S, out, cnt,
-                                                    one_chunk ? nullptr : L.work, cap, width);
+    k<<<(int)(one_chunk ? blocks : resident), TB, 0, s>>>(T, R.org, R.dir, R.root, R.order, R.n, S, out, cnt,
+                                                    one_chunk ? nullptr : L.work, cap, width, V);
 }
 
 template <int SMAX, bool SHORT, bool SKIP, bool COUNT, bool WOOP>
@@ -1173,6 +1211,29 @@ float4 *woop_tris(pm_ctx *ctx, int tris, hipStream_t s) {
     return W;
 }
 
+void query_cus(pm_ctx *ctx) {
+    if (ctx->num_cus) return;
+    int v = 0;
+    PM_HIP(hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, ctx->device));
+    ctx->num_cus = v > 0 ? v : 1;
+}
+
+template <int SMAX, bool SHORT, bool SKIP, bool WOOP>
+void launch_canvas_coop(const TreeDev &T, const RayBatch &R, int S, const Launch &L, hipStream_t s,
+                        const CanvasArgs &V) {
+    auto k = trace_coop_kernel<SMAX, SHORT, SKIP, false, false, WOOP, true>;
+    launch_coop(k, T, R, S, nullptr, nullptr, L, 0, s, V);
+}
+
+template <bool SKIP, bool WOOP>
+void dispatch_canvas(const TreeDev &T, int algo, const RayBatch &R, int S, const Launch &L, hipStream_t s,
+                     const CanvasArgs &V) {
+    if (algo == PM_TRACE_KD_RESTART) launch_canvas_coop<1, false, SKIP, WOOP>(T, R, 1, L, s, V);
+    else if (S <= 4) launch_canvas_coop<4, true, SKIP, WOOP>(T, R, S, L, s, V);
+    else if (S <= 8) launch_canvas_coop<8, true, SKIP, WOOP>(T, R, S, L, s, V);
+    else launch_canvas_coop<16, true, SKIP, WOOP>(T, R, S, L, s, V);
+}
+
 template <int ALGO>
 void launch_canvas(bool skip, bool woop, int blocks, hipStream_t s, const TreeDev &T, const float4 *A,
                    const float4 *B, const float4 *C, int ntris, const float4 *org, const float4 *dir, int n,
@@ -1218,11 +1279,7 @@ void trace_rays(pm_ctx *ctx, int algo, const float4 *org, const float4 *dir, int
     RayBatch R{org, dir, ray_mesh, nullptr, nrays};
     if (ray_order_applies(prm, nrays))
         R.order = ray_order(ctx, org, dir, ray_mesh, nrays, s, ext ? &ext->order : nullptr);
-    if (!ctx->num_cus) {
-        int v = 0;
-        PM_HIP(hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, ctx->device));
-        ctx->num_cus = v > 0 ? v : 1;
-    }
+    query_cus(ctx);
     int *work = nullptr;
     if (ext) {
         work = ext->work;
@@ -1260,7 +1317,16 @@ void trace_canvas(pm_ctx *ctx, int algo, const float4 *org, const float4 *dir, i
     } else {
         if (woop) T.leaf_woop = woop_slots(ctx, s);
         const bool skip = prm.leaf_skipping && ctx->has_boxes;
-        if (algo == PM_TRACE_KD_RESTART)
+        if (48ll * T.num_slots < (1ll << 32)) {
+            query_cus(ctx);
+            const Launch W{ctx->num_cus, nullptr, 0};
+            const RayBatch R{org, dir, nullptr, nullptr, nrays};
+            const CanvasArgs V{n0, n1, n2, c0, L, max_bounces, canvas};
+            if (skip && woop) dispatch_canvas<true, true>(T, algo, R, prm.stack_size, W, s, V);
+            else if (skip) dispatch_canvas<true, false>(T, algo, R, prm.stack_size, W, s, V);
+            else if (woop) dispatch_canvas<false, true>(T, algo, R, prm.stack_size, W, s, V);
+            else dispatch_canvas<false, false>(T, algo, R, prm.stack_size, W, s, V);
+        } else if (algo == PM_TRACE_KD_RESTART)
             launch_canvas<PM_TRACE_KD_RESTART>(skip, woop, blocks, s, T, A, B, C, 0, org, dir, nrays, 1, n0, n1, n2,
                                                c0, L, max_bounces, canvas);
         else

@@ -67,3 +67,27 @@ def test_root_leaf_bit_exact(pm, orc, scenes, torch, ntris, boxes):
         h = pm.hits_to_numpy(ctx.trace(algo, dev(torch, org), dev(torch, dirs), pm.trace_params()))
         assert_same_hits(h, want, f"{ntris} triangles, algo {algo}")
     ctx.close()
+
+
+@pytest.mark.parametrize("algo,stack", [("SHORT_STACK", 1), ("SHORT_STACK", 5), ("SHORT_STACK", 13), ("KD_RESTART", 4)])
+@pytest.mark.parametrize("woop", [False, True])
+def test_canvas_ray_counts_bit_exact(pm, orc, scenes, torch, algo, stack, woop):
+    """canvas bytes at ray counts that fill part of a wave, one and many, and at
+    bounce limits met by some rays"""
+    from test_gpu_extras import shading_scene
+    tris, _, normals, col, light = shading_scene(scenes)
+    org, dirs = scenes.pinhole_rays(300, 240, (0.0, 0.0, 3.5), (0.0, 0.0, 0.0), fov_deg=45.0, seed=9)
+    test = pm.WOOP if woop else pm.MOELLER
+    ctx = pm.Context(0)
+    ctx.build(*[dev(torch, t) for t in tris], pm.build_params("reference"))
+    ref = orc.build(tris, orc.build_params("reference"))
+    a = getattr(pm, algo)
+    N, C = [dev(torch, x) for x in normals], dev(torch, col)
+    for n, bounces in ((1, 64), (63, 64), (65, 1), (7001, 3), (72000, 64), (72000, 2)):
+        o, d = org[-n:].copy(), dirs[-n:].copy()
+        got = ctx.trace_canvas(a, dev(torch, o), dev(torch, d), N, C, light, max_bounces=bounces,
+                               params=pm.trace_params(stack_size=stack, intersection=test)).cpu().numpy()
+        want = orc.trace_canvas(ref, tris, o, d, a, normals, col, light, max_bounces=bounces, stack_size=stack,
+                                threads=8, intersection=test)
+        assert np.array_equal(got, want), (n, bounces, np.nonzero((got != want).any(1))[0][:5])
+    ctx.close()
