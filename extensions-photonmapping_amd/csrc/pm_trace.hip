@@ -811,43 +811,242 @@ __global__ __launch_bounds__(TB) void trace_coop_kernel(TreeDev T, const float4 
     }
 }
 
-// Brute force: every lane tests every triangle in index order; triangles are
-// staged through LDS one tile at a time (one tile = TB triangles, 12 KiB).
-// WOOP: P0/P1/P2 are the triangles' Woop matrices m0/m1/m2 instead
-template <bool COUNT, bool WOOP>
-__global__ __launch_bounds__(TB) void brute_kernel(const float4 *__restrict__ P0,
-                                                   const float4 *__restrict__ P1,
-                                                   const float4 *__restrict__ P2, int ntris,
-                                                   const float4 *__restrict__ org,
-                                                   const float4 *__restrict__ dir, int n,
-                                                   pm_hit *__restrict__ out,
-                                                   int4 *__restrict__ counters) {
-    __shared__ float4 s0[TB], s1[TB], s2[TB];
-    const int r = blockIdx.x * TB + threadIdx.x;
-    const bool live = r < n;
-    f3 o = {0.0f, 0.0f, 0.0f}, d = {0.0f, 0.0f, 1.0f};
-    if (live) { o = mk3(org[r]); d = mk3(dir[r]); }
+// ---- brute force
+// Every ray against every triangle; the record is the one the sequential loop
+// ends with (accept 0 <= t <= th, then th = t): the smallest t, ties to the
+// highest index, so hits are offered as keys (t bits, ~index) to the ray's
+// 64-bit LDS minimum and the winner is tested once more for t, u, v.
+//
+// Moller-Trumbore: nearly all of the work is to find that a ray passes a
+// triangle by, and that is a contraction.  With w = o x d and N = e1 x e2,
+//   det = -d.N,  f1 = det u = d.(v0 x e2) + w.e2,
+//   f2 = det v = -d.(v0 x e1) - w.e1,  f3 = det - f1 - f2,
+// so the three edge values of 32 triangles and 32 rays are three 32x32x8
+// matrix products of (d, w) with the triangles' vectors.  A pair the exact
+// test accepts has f1, f2, f3 of one sign up to rounding; pairs that do not
+// (beyond a bound E on every rounding involved) are dropped, the others are
+// listed and tested exactly, 64 at a time.
+//
+// The bound.  Coordinates are taken relative to c, a vertex (exact to half an
+// ulp of the differences), and scaled by S > 0:
+//   ray       (S d, w) / alpha,          alpha = |d| (S + |o|)
+//   triangle  (g / S, h) / beta,         beta = em (S + V) / S,
+//             em = |e1| + |e2|, V = |v0| + em, g / h its d and w vectors
+// The halves of the ray's vector then have norms S / (S + |o|) and |o| / (S +
+// |o|), the triangle's at most V / (S + V) and S / (S + V), so the sum of the
+// absolute products of a value is at most S (|o| + V) / ((S + |o|) (S + V)) <=
+// 1, and alpha beta >= |d| em (|o| + V).  Rounding the entries to 16 bits moves
+// a value by at most 2^-10 (2^-11 of an entry on either side) and, where
+// entries are tiny or flushed (2^-14 of each), by 2 sqrt(3) 2^-14 = 0.00021;
+// the exact test's own rounding of f1, f2, det (a few 2^-24 of |d| em (|o| +
+// V)), of u + v <= 1 and of these vectors is below 2^-18.  E = 0.00122 covers
+// their sum, 0.00119.
+// A ray or triangle whose alpha or beta is not in [2^-40, 2^40] (NaN,
+// infinite, degenerate or out of range) gets the zero vector: always listed.
+//
+constexpr int BRUTE_WAVES = 16;          // waves of a block, each with its share of the triangles
+constexpr int BRUTE_T = 64 * BRUTE_WAVES;
+constexpr float BRUTE_E = 0x1.4p-10f;
+
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ float norm3(f3 a) { return sqrtf(dot3(a, a)); }
+__device__ __forceinline__ bool brute_scale_ok(float x) { return x >= 0x1p-40f && x <= 0x1p40f; }
+__device__ __forceinline__ half4 to_half4(f3 a) {
+    half4 h;
+    h.x = (_Float16)a.x; h.y = (_Float16)a.y; h.z = (_Float16)a.z; h.w = (_Float16)0.0f;
+    return h;
+}
+
+__device__ __forceinline__ unsigned long long hit_key(float t, int id) {
+    return ((unsigned long long)__float_as_uint(t + 0.0f) << 32) | (unsigned)~id;
+}
+
+// the record of a ray whose best key is k: the winner's own test again
+template <bool WOOP>
+__device__ __forceinline__ pm_hit brute_record(unsigned long long k, const float4 *__restrict__ A,
+                                               const float4 *__restrict__ B, const float4 *__restrict__ C, f3 o,
+                                               f3 d) {
+    pm_hit res = miss_record();
+    if (k == ~0ull) return res;
+    const int id = (int)~(unsigned)(k & 0xffffffffu);
     float th = F_INF, tu = 0.0f, tv = 0.0f;
-    int hit = -1;
-    for (int base = 0; base < ntris; base += TB) {
-        const int k = base + threadIdx.x;
-        __syncthreads();
-        if (k < ntris) { s0[threadIdx.x] = P0[k]; s1[threadIdx.x] = P1[k]; s2[threadIdx.x] = P2[k]; }
-        __syncthreads();
-        const int m = min(TB, ntris - base);
-        if (live) {
-            for (int j = 0; j < m; ++j) {
-                const bool h = WOOP ? woop_test(s0[j], s1[j], s2[j], o, d, th, tu, tv)
-                                    : moller_trumbore(mk3(s0[j]), mk3(s1[j]), mk3(s2[j]), o, d, th, tu, tv);
-                if (h) hit = base + j;
+    const bool h = WOOP ? woop_test(A[id], B[id], C[id], o, d, th, tu, tv)
+                        : moller_trumbore(mk3(A[id]), mk3(B[id]), mk3(C[id]), o, d, th, tu, tv);
+    if (h && th < F_INF) { res.id = id; res.t = th; res.u = tu; res.v = tv; }
+    return res;
+}
+
+// RT: 32-ray tiles of a block (the same rays for its 16 waves, which take the
+// triangle tiles w, w + 16, ...)
+template <int RT, bool COUNT>
+__global__ __launch_bounds__(BRUTE_T) void brute_kernel(const float4 *__restrict__ P0, const float4 *__restrict__ P1,
+                                                        const float4 *__restrict__ P2, int ntris,
+                                                        const float4 *__restrict__ org,
+                                                        const float4 *__restrict__ dir, int n,
+                                                        pm_hit *__restrict__ out, int4 *__restrict__ counters) {
+    constexpr int NR = 32 * RT;
+    __shared__ unsigned long long key[NR];
+    __shared__ int list_tri[BRUTE_WAVES][128];
+    __shared__ unsigned short list_ray[BRUTE_WAVES][128];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 31;
+    const bool wpart = lane >= 32;         // lanes 32..63 hold the operands' w half (k = 4..7)
+    const int r0 = blockIdx.x * NR;
+    for (int j = threadIdx.x; j < NR; j += BRUTE_T) key[j] = ~0ull;
+    __syncthreads();
+    if (ntris > 0) {
+        // the frame: c a vertex, S the size of a sample of the triangles
+        // (any c and any S > 0 are right; these keep E small in the scene)
+        const f3 first = mk3(P0[0]);
+        const bool fin = fabsf(first.x) < 0x1p40f && fabsf(first.y) < 0x1p40f && fabsf(first.z) < 0x1p40f;
+        const f3 c = fin ? first : f3{0.0f, 0.0f, 0.0f};
+        float S;
+        {
+            const int k = (int)((long long)lane * ntris / 64);
+            float v = norm3(sub3(mk3(P0[k]), c));
+            v = brute_scale_ok(v) ? v : 0.0f;
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
+            S = v > 0.0f ? v : 1.0f;
+        }
+        half4 rays[RT];
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            const int r = min(r0 + 32 * t + col, n - 1);
+            const f3 o = sub3(mk3(org[r]), c), d = mk3(dir[r]);
+            const float alpha = norm3(d) * (S + norm3(o));
+            const f3 x = wpart ? cross3(o, d) : f3{d.x * S, d.y * S, d.z * S};
+            const float k = 1.0f / alpha;
+            rays[t] = to_half4(brute_scale_ok(alpha) ? f3{x.x * k, x.y * k, x.z * k} : f3{0.0f, 0.0f, 0.0f});
+        }
+        int pending = 0;
+        // tests the list's first m pairs exactly
+        auto flush = [&](int m) {
+            if (lane < m) {
+                const int tri = list_tri[w][lane], j = list_ray[w][lane];
+                float th = F_INF, tu, tv;
+                if (moller_trumbore(mk3(P0[tri]), mk3(P1[tri]), mk3(P2[tri]), mk3(org[r0 + j]), mk3(dir[r0 + j]), th,
+                                    tu, tv))
+                    atomicMin(&key[j], hit_key(th, tri));
+            }
+        };
+        const int tiles = (ntris + 31) >> 5;
+        auto load_tri = [&](int tile, float4 &a, float4 &b, float4 &e) {
+            const int k = min(32 * tile + col, ntris - 1);
+            a = P0[k]; b = P1[k]; e = P2[k];
+        };
+        float4 na, nb, ne;
+        if (w < tiles) load_tri(w, na, nb, ne);
+        for (int tile = w; tile < tiles; tile += BRUTE_WAVES) {
+            const f3 p0 = mk3(na), p1 = mk3(nb), p2 = mk3(ne);
+            if (tile + BRUTE_WAVES < tiles) load_tri(tile + BRUTE_WAVES, na, nb, ne);
+            half4 t1, t2, t3;
+            {
+                const f3 v0 = sub3(p0, c), e1 = sub3(p1, p0), e2 = sub3(p2, p0);
+                const float em = norm3(e1) + norm3(e2);
+                const float beta = em * (S + norm3(v0) + em) / S;
+                const bool ok = brute_scale_ok(beta);
+                f3 g1, g2, g3;
+                float k = 1.0f / beta;
+                if (wpart) {
+                    g1 = e2; g2 = {-e1.x, -e1.y, -e1.z}; g3 = sub3(e1, e2);
+                } else {
+                    k = k / S;
+                    g1 = cross3(v0, e2);
+                    g2 = cross3(e1, v0);
+                    const f3 m = cross3(e2, e1);
+                    g3 = sub3(sub3(m, g1), g2);
+                }
+                k = ok ? k : 0.0f;
+                auto scaled = [&](f3 g) {
+                    return to_half4(ok ? f3{g.x * k, g.y * k, g.z * k} : f3{0.0f, 0.0f, 0.0f});
+                };
+                t1 = scaled(g1); t2 = scaled(g2); t3 = scaled(g3);
+            }
+#pragma unroll
+            for (int t = 0; t < RT; ++t) {
+                const f32x16 zero = {0};
+                const f32x16 f1 = __builtin_amdgcn_mfma_f32_32x32x8f16(t1, rays[t], zero, 0, 0, 0);
+                const f32x16 f2 = __builtin_amdgcn_mfma_f32_32x32x8f16(t2, rays[t], zero, 0, 0, 0);
+                const f32x16 f3_ = __builtin_amdgcn_mfma_f32_32x32x8f16(t3, rays[t], zero, 0, 0, 0);
+                // max over the tile of max(min f, -max f): a pair is listed at >= -E
+                float best = -1.0f;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float lo = fminf(fminf(f1[r], f2[r]), f3_[r]), hi = fmaxf(fmaxf(f1[r], f2[r]), f3_[r]);
+                    best = fmaxf(fmaxf(best, lo), -hi);
+                }
+                if (__ballot(best >= -BRUTE_E) == 0ull) continue;
+                const bool ray_in = r0 + 32 * t + col < n;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float lo = fminf(fminf(f1[r], f2[r]), f3_[r]), hi = fmaxf(fmaxf(f1[r], f2[r]), f3_[r]);
+                    const int tri = 32 * tile + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                    const bool cand = fmaxf(lo, -hi) >= -BRUTE_E && ray_in && tri < ntris;
+                    const unsigned long long m = __ballot(cand);
+                    if (m == 0ull) continue;
+                    if (cand) {
+                        const int at = pending + __popcll(m & (lane ? ~0ull >> (64 - lane) : 0ull));
+                        list_tri[w][at] = tri;
+                        list_ray[w][at] = (unsigned short)(32 * t + col);
+                    }
+                    pending += __popcll(m);
+                    if (pending >= 64) {
+                        wave_sync();
+                        flush(64);
+                        wave_sync();
+                        pending -= 64;
+                        if (lane < pending) {
+                            list_tri[w][lane] = list_tri[w][64 + lane];
+                            list_ray[w][lane] = list_ray[w][64 + lane];
+                        }
+                        wave_sync();
+                    }
+                }
             }
         }
+        wave_sync();
+        flush(pending);
     }
-    if (!live) return;
-    pm_hit res = miss_record();
-    if (th < F_INF && hit != -1) { res.id = hit; res.t = th; res.u = tu; res.v = tv; }
-    out[r] = res;
-    if (COUNT) counters[r] = make_int4(0, 0, ntris, 0);
+    __syncthreads();
+    for (int j = threadIdx.x; j < NR; j += BRUTE_T) {
+        const int r = r0 + j;
+        if (r >= n) continue;
+        out[r] = brute_record<false>(key[j], P0, P1, P2, mk3(org[r]), mk3(dir[r]));
+        if (COUNT) counters[r] = make_int4(0, 0, ntris, 0);
+    }
+}
+
+// Woop: P0/P1/P2 hold the matrices m0/m1/m2.  64 rays a block, every wave
+// with its share of the triangles (w, w + 16, ...), read through the scalar
+// cache: one triangle for the 64 lanes.  (The matrices come out of a float
+// inversion, so no bound of their test's rounding is small enough to filter by.)
+template <bool COUNT>
+__global__ __launch_bounds__(BRUTE_T) void brute_woop_kernel(const float4 *__restrict__ W0,
+                                                             const float4 *__restrict__ W1,
+                                                             const float4 *__restrict__ W2, int ntris,
+                                                             const float4 *__restrict__ org,
+                                                             const float4 *__restrict__ dir, int n,
+                                                             pm_hit *__restrict__ out, int4 *__restrict__ counters) {
+    __shared__ unsigned long long key[64];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (threadIdx.x < 64) key[threadIdx.x] = ~0ull;
+    __syncthreads();
+    const int r = blockIdx.x * 64 + lane;
+    const f3 o = mk3(org[min(r, n - 1)]), d = mk3(dir[min(r, n - 1)]);
+    float th = F_INF, tu = 0.0f, tv = 0.0f;
+    int hit = -1;
+#pragma unroll 2
+    for (int k = w; k < ntris; k += BRUTE_WAVES)
+        if (woop_test(W0[k], W1[k], W2[k], o, d, th, tu, tv)) hit = k;
+    if (hit >= 0) atomicMin(&key[lane], hit_key(th, hit));
+    __syncthreads();
+    if (w == 0 && r < n) {
+        out[r] = brute_record<true>(key[lane], W0, W1, W2, o, d);
+        if (COUNT) counters[r] = make_int4(0, 0, ntris, 0);
+    }
 }
 
 // ---- trace view
@@ -1211,6 +1410,27 @@ float4 *woop_tris(pm_ctx *ctx, int tris, hipStream_t s) {
     return W;
 }
 
+void query_cus(pm_ctx *ctx);
+
+// More rays a block mean fewer conversions of the triangles' vectors per pair,
+// fewer rays more blocks: the most that still give every CU a block.  65,536
+// rays x 5,316 triangles: 109 us with 128 rays a block, 134 with 64, 187 with
+// 32 (256 need more registers than four waves a SIMD leave); the kernel it
+// replaced, every ray's exact test against every triangle in 1,024 waves, 1,440.
+// Bound by VALU issue: three instructions per pair and matrix tile row.
+template <bool COUNT>
+void brute_rays(pm_ctx *ctx, int tris, const float4 *org, const float4 *dir, int n, pm_hit *out, int4 *counters,
+                hipStream_t s) {
+    query_cus(ctx);
+    auto launch = [&](auto k, int rays) {
+        k<<<(n + rays - 1) / rays, BRUTE_T, 0, s>>>(ctx->p0, ctx->p1, ctx->p2, tris, org, dir, n, out, counters);
+    };
+    const long long per_cu = (long long)n / ctx->num_cus;
+    if (per_cu >= 128) launch(brute_kernel<4, COUNT>, 128);
+    else if (per_cu >= 64) launch(brute_kernel<2, COUNT>, 64);
+    else launch(brute_kernel<1, COUNT>, 32);
+}
+
 void query_cus(pm_ctx *ctx) {
     if (ctx->num_cus) return;
     int v = 0;
@@ -1258,16 +1478,19 @@ void trace_rays(pm_ctx *ctx, int algo, const float4 *org, const float4 *dir, int
     const bool woop = prm.intersection == PM_INTERSECT_WOOP;
     if (algo == PM_TRACE_BRUTE) {
         const int tris = prm.brute_cap > 0 ? std::min(ctx->ntris, prm.brute_cap) : ctx->ntris;
-        const int blocks = (nrays + TB - 1) / TB;
-        const float4 *A = ctx->p0, *B = ctx->p1, *C = ctx->p2;
         if (woop) {
             const float4 *W = woop_tris(ctx, tris, s);
-            A = W; B = W + tris; C = W + 2ll * tris;
-            if (counters) brute_kernel<true, true><<<blocks, TB, 0, s>>>(A, B, C, tris, org, dir, nrays, out, counters);
-            else brute_kernel<false, true><<<blocks, TB, 0, s>>>(A, B, C, tris, org, dir, nrays, out, counters);
+            const int blocks = (nrays + 63) / 64;
+            if (counters)
+                brute_woop_kernel<true><<<blocks, BRUTE_T, 0, s>>>(W, W + tris, W + 2ll * tris, tris, org, dir, nrays,
+                                                                  out, counters);
+            else
+                brute_woop_kernel<false><<<blocks, BRUTE_T, 0, s>>>(W, W + tris, W + 2ll * tris, tris, org, dir,
+                                                                   nrays, out, counters);
+        } else if (counters) {
+            brute_rays<true>(ctx, tris, org, dir, nrays, out, counters, s);
         } else {
-            if (counters) brute_kernel<true, false><<<blocks, TB, 0, s>>>(A, B, C, tris, org, dir, nrays, out, counters);
-            else brute_kernel<false, false><<<blocks, TB, 0, s>>>(A, B, C, tris, org, dir, nrays, out, counters);
+            brute_rays<false>(ctx, tris, org, dir, nrays, out, counters, s);
         }
         PM_LAUNCH_CHECK();
         return;
