@@ -1429,9 +1429,28 @@ __global__ void propagate_parent_kernel(NodePtrs N, const int *__restrict__ leaf
 }
 
 // ------------------------------------------------------------------ lower
+// PRIM_SLOTS counters of the lower levels' prims: each wave of the screen
+// pass adds to slot (wave index % PRIM_SLOTS), so the adds do not queue on one
+// word; plan_lower_kernel folds them into the level state
+constexpr int PRIM_SLOTS = 64;
+
+// the lower levels' start, by the first block of the pass that prepares their
+// nodes (it changes nothing that pass reads): the upper leaves are the list
+__device__ __forceinline__ void plan_lower_start(Lvl *L, unsigned long long *parts) {
+    if (blockIdx.x == 0 && threadIdx.x < PRIM_SLOTS) parts[threadIdx.x] = 0ull;
+    if (threadIdx.x | blockIdx.x) return;
+    L->An = L->status ? 0 : L->nleaf;
+    L->use_list = 1;
+    L->list_base = 0;
+    L->lower_levels = 0;
+    L->cand_n = 0;
+}
+
 // PreprocessLeafNodes (TriangleMapBitmapCreator.cu:32-49)
-__global__ void bitmap_leaves_kernel(NodePtrs N, const int *__restrict__ leaf_ids, const Lvl *__restrict__ L) {
+__global__ void bitmap_leaves_kernel(NodePtrs N, const int *__restrict__ leaf_ids, Lvl *__restrict__ L,
+                                     unsigned long long *parts) {
     const int n = L->status ? 0 : L->nleaf;
+    if (parts) plan_lower_start(L, parts);
     GRID_STRIDE(i, n) {
         const int leaf = leaf_ids[i];
         N.info[leaf] = LEAF;
@@ -1442,9 +1461,10 @@ __global__ void bitmap_leaves_kernel(NodePtrs N, const int *__restrict__ leaf_id
 
 // PreprocesLowerNodes (LowerTriangleMap.h:56-81); starts the lower levels
 // with the upper leaves as the node list
-__global__ void lower_prep_kernel(NodePtrs N, const int *__restrict__ leaf_ids, const Lvl *__restrict__ L,
-                                  const float *__restrict__ areas) {
+__global__ void lower_prep_kernel(NodePtrs N, const int *__restrict__ leaf_ids, Lvl *__restrict__ L,
+                                  const float *__restrict__ areas, unsigned long long *parts) {
     const int n = L->status ? 0 : L->nleaf;
+    plan_lower_start(L, parts);
     GRID_STRIDE(i, n) {
         const int leaf = leaf_ids[i];
         const int pi = N.prim_index[leaf];
@@ -1460,21 +1480,6 @@ __global__ void lower_prep_kernel(NodePtrs N, const int *__restrict__ leaf_ids, 
         N.area[leaf] = a;
         N.bitmap[leaf] = (long long)bmp;
     }
-}
-
-// PRIM_SLOTS counters of the lower levels' prims: each wave of the screen
-// pass adds to slot (wave index % PRIM_SLOTS), so the adds do not queue on one
-// word; plan_lower_kernel folds them into the level state
-constexpr int PRIM_SLOTS = 64;
-
-__global__ void plan_lower_start_kernel(Lvl *L, unsigned long long *parts) {
-    if (blockIdx.x == 0 && threadIdx.x < PRIM_SLOTS) parts[threadIdx.x] = 0ull;
-    if (threadIdx.x | blockIdx.x) return;
-    L->An = L->status ? 0 : L->nleaf;
-    L->use_list = 1;
-    L->list_base = 0;
-    L->lower_levels = 0;
-    L->cand_n = 0;
 }
 
 // Exact early rejection for the SAH decision.  Every candidate plane puts
@@ -1814,12 +1819,24 @@ __device__ __forceinline__ unsigned long long lane_u64(unsigned long long v, int
     return ((unsigned long long)hi << 32) | lo;
 }
 
-// First pass of a lower level: a wave takes 64 nodes at a time, one per lane.
+// Nodes a wave of the screen pass takes at a time: 64 where that still gives
+// SCREEN_WAVES waves, fewer (down to one pair) on smaller levels.  A wave
+// decides its nodes one pair after another (about 0.8 us a pair), so 547 nodes
+// at 64 a wave took 54 us in 9 waves and 5 us at 2 a wave; at 130,000 nodes 64
+// and 32 a wave are equal, and fewer cost more than they hide.
+constexpr int SCREEN_WAVES = 1024;
+__host__ __device__ inline int screen_nodes(long long An) {
+    int k = 64;
+    while (k > 2 && An < (long long)SCREEN_WAVES * k) k >>= 1;
+    return k;
+}
+
+// First pass of a lower level: a wave takes up to 64 nodes at a time, one per lane.
 // Nodes with leaf cost <= 0 (n <= C_t: costs are >= 0, no split can win)
 // become leaves lane by lane; the others get the exact bound of
 // sah_cannot_split one node at a time, with the next node's areas already in
-// flight.  Nodes the bound cannot settle (and nodes forced to split) are
-// listed for sah_kernel, one list append per wave and batch.  Each node's
+// flight.  Nodes the bound cannot settle (and, untried, nodes forced to split)
+// are listed for sah_kernel, one list append per wave and batch.  Each node's
 // decision is its own, so the list order does not matter.
 __global__ __launch_bounds__(WPB * 64) void sah_screen_kernel(
     NodePtrs N, const int *__restrict__ leaf_ids, Lvl *__restrict__ L, const float *__restrict__ areas,
@@ -1828,9 +1845,10 @@ __global__ __launch_bounds__(WPB * 64) void sah_screen_kernel(
     const int An = L->An, list_base = L->list_base;
     const int *list = L->use_list ? leaf_ids : nullptr;
     const int lane = threadIdx.x & 63;
-    for (int base = wave_index() * 64; base < An; base += wave_count() * 64) {
+    const int npw = screen_nodes(An);
+    for (int base = wave_index() * npw; base < An; base += wave_count() * npw) {
         const int id = base + lane;
-        const bool valid = id < An;
+        const bool valid = lane < npw && id < An;
         int par = 0, pi = 0;
         unsigned long long bmp = 0ull;
         float nodeA = 0.0f;
@@ -1843,14 +1861,14 @@ __global__ __launch_bounds__(WPB * 64) void sah_screen_kernel(
         const int n = __popcll(bmp);
         const bool forced = leaf_max > 0 && n > leaf_max;
         const float leaf_cost = ((float)n - Ct) * nodeA;
-        unsigned long long m = __ballot(valid && (forced || leaf_cost > 0.0f));
+        unsigned long long m = __ballot(valid && !forced && leaf_cost > 0.0f);
         {   // work count: the batch's prims
             int t = n;
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
             if (lane == 0) atomicAdd(&parts[wave_index() % PRIM_SLOTS], (unsigned long long)t);
         }
-        unsigned long long search = 0ull;
+        unsigned long long search = __ballot(valid && forced);   // no bound to try: searched
         // the nodes of m in groups: two nodes, one per half-wave, when both
         // bitmaps fit in bits 0..31 (k2 >= 0), else one node on the whole wave
         auto group = [&](unsigned long long mm, int &k1, int &k2) {
@@ -1892,18 +1910,16 @@ __global__ __launch_bounds__(WPB * 64) void sah_screen_kernel(
             }
             const unsigned long long kb = lane_u64(bmp, k1);
             const int kn = __popcll(kb);
-            const bool kforced = leaf_max > 0 && kn > leaf_max;
             if (k2 < 0) {
-                if (kforced || !sah_cannot_split(kb, a, kn, bonus, lane_float(leaf_cost, k1))) search |= 1ull << k1;
+                if (!sah_cannot_split(kb, a, kn, bonus, lane_float(leaf_cost, k1))) search |= 1ull << k1;
             } else {
                 const unsigned long long kb2 = lane_u64(bmp, k2);
                 const int kn2 = __popcll(kb2);
-                const bool kforced2 = leaf_max > 0 && kn2 > leaf_max;
                 const bool r = sah_cannot_split_pair(kb, kb2, a, kn, kn2, bonus, lane_float(leaf_cost, k1),
                                                      lane_float(leaf_cost, k2));
                 const unsigned long long rb = __ballot(r);
-                if (kforced || !(rb & 1ull)) search |= 1ull << k1;
-                if (kforced2 || !((rb >> 32) & 1ull)) search |= 1ull << k2;
+                if (!(rb & 1ull)) search |= 1ull << k1;
+                if (!((rb >> 32) & 1ull)) search |= 1ull << k2;
             }
             k1 = nk1;
             k2 = nk2;
@@ -2003,14 +2019,13 @@ __global__ __launch_bounds__(WPB * 64) void balanced_kernel(
 }
 
 // after the SAH pass: place the split nodes' children (c: the level's prims)
-__device__ void plan_lower_apply(Lvl *L, const int *__restrict__ off, unsigned long long c) {
+__device__ void plan_lower_apply(Lvl *L, int splits, unsigned long long c) {
     L->lower_prims += c;
     const int An = L->An;
     L->splits = 0;
     if (An == 0) return;
     L->lower_levels += 1;
     L->seen_lower = max(L->seen_lower, (long long)An);
-    const int splits = off[An];
     if ((long long)L->nodes_size + 2ll * splits > L->cap_nodes || 2 * splits > L->cap_lower) {
         lvl_fail(L, PM_ERR_CAPACITY);
         return;
@@ -2020,28 +2035,67 @@ __device__ void plan_lower_apply(Lvl *L, const int *__restrict__ off, unsigned l
     L->nodes_size += 2 * splits;
 }
 
-// one block of 64 threads; an eager build (mirror) also publishes the state
-__global__ void plan_lower_kernel(Lvl *L, const int *__restrict__ off, unsigned long long *parts,
-                                  LvlMirror::Rec *mirror, unsigned seq) {
-    if (blockIdx.x) return;
-    // the screen pass's prim counts (one wave of PRIM_SLOTS threads)
-    unsigned long long c = threadIdx.x < PRIM_SLOTS ? parts[threadIdx.x] : 0ull;
-    if (threadIdx.x < PRIM_SLOTS) parts[threadIdx.x] = 0ull;
+// The plan of a lower level, one block: the children's offsets (SCAN: the
+// exclusive scan of the split flags, for levels of up to PLAN_SCAN nodes; else
+// scanned before), their place among the nodes, and the next level, which is
+// those children (the children pass reads this level's list from ch_*).  An
+// eager build (mirror) also publishes the state.
+// Scan, plan and advance as launches of their own were 8 us a level and the
+// gaps between them; a level of more nodes is scanned by more than one block.
+constexpr int PLAN_T = 1024, PLAN_SCAN = 4 * 4 * PLAN_T;
+template <bool SCAN>
+__global__ __launch_bounds__(PLAN_T) void plan_lower_kernel(Lvl *L, const int *__restrict__ flag,
+                                                            int *__restrict__ off, unsigned long long *parts,
+                                                            LvlMirror::Rec *mirror, unsigned seq) {
+    __shared__ int wsum[PLAN_T / 64];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int An = L->An;
+    int total = 0;
+    if (SCAN) {
+        for (int base = 0; base < An; base += 4 * PLAN_T) {
+            const int i = base + 4 * t;
+            int v[4], sum = 0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                v[j] = i + j < An ? flag[i + j] : 0;
+                sum += v[j];
+            }
+            const int incl = wave_incl_scan(sum);
+            if (lane == 63) wsum[w] = incl;
+            __syncthreads();
+            int run = total + incl - sum;
+            for (int j = 0; j < PLAN_T / 64; ++j) {
+                const int x = wsum[j];
+                if (j < w) run += x;
+                total += x;
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (i + j < An) off[i + j] = run;
+                run += v[j];
+            }
+            __syncthreads();
+        }
+    }
+    // the screen pass's prim counts (the first wave)
+    unsigned long long c = t < PRIM_SLOTS ? parts[t] : 0ull;
+    if (t < PRIM_SLOTS) parts[t] = 0ull;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
-    if (threadIdx.x == 0) plan_lower_apply(L, off, c);
+    if (t == 0) {
+        if (!SCAN && An > 0) total = off[An];
+        L->ch_An = An;
+        L->ch_list_base = L->list_base;
+        L->ch_use_list = L->use_list;
+        plan_lower_apply(L, total, c);
+        L->An = 2 * L->splits;
+        L->use_list = 0;
+        L->list_base = L->lower_base;
+        L->cand_n = 0;
+    }
     if (!mirror) return;
     __syncthreads();
     publish_level(L, mirror, seq);
-}
-
-// after the children: the next lower level is the new children
-__global__ void plan_lower_advance_kernel(Lvl *L) {
-    if (threadIdx.x | blockIdx.x) return;
-    L->An = 2 * L->splits;
-    L->use_list = 0;
-    L->list_base = L->lower_base;
-    L->cand_n = 0;
 }
 
 // CreateLowerSAHChildren (LowerTriangleMap.h:557-600) + PropagateAabbToChildren
@@ -2083,9 +2137,9 @@ __device__ __forceinline__ void lower_children_node(const NodePtrs &N, int id, i
 __global__ void lower_children_kernel(NodePtrs N, const int *__restrict__ leaf_ids, const Lvl *__restrict__ L,
                                       int propagate, const int *__restrict__ flag, const int *__restrict__ off,
                                       const long long *__restrict__ sets, const float *__restrict__ careas) {
-    const int An = L->splits > 0 ? L->An : 0, list_base = L->list_base;
+    const int An = L->splits > 0 ? L->ch_An : 0, list_base = L->ch_list_base;
     const int base = L->lower_base, splits = L->splits;
-    const int *list = L->use_list ? leaf_ids : nullptr;
+    const int *list = L->ch_use_list ? leaf_ids : nullptr;
     GRID_STRIDE(id, An) {
         if (!flag[id]) continue;
         const int par = list ? list[id] : list_base + id;
@@ -2483,26 +2537,25 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
 
     // lower stage
     const bool balanced = prm.lower_algorithm == PM_LOWER_BALANCED;
+    if (sah && !graph) sc.prims_part.reserve(PRIM_SLOTS, s);
+    unsigned long long *const parts = sah ? sc.prims_part.ptr : nullptr;
     if (!sah || balanced) {   // PreprocessLeafNodes: counts -> masks
-        bitmap_leaves_kernel<<<grid_for(nlf, BS, graph ? 4096 : INT_MAX), BS, 0, s>>>(NP, ctx->leaf_ids.ptr, L);
+        bitmap_leaves_kernel<<<grid_for(nlf, BS, graph ? 4096 : INT_MAX), BS, 0, s>>>(NP, ctx->leaf_ids.ptr, L, parts);
+        PM_LAUNCH_CHECK();
+    } else {
+        lower_prep_kernel<<<grid_for(nlf, BS, graph ? 4096 : INT_MAX), BS, 0, s>>>(NP, ctx->leaf_ids.ptr, L,
+                                                                                   sc.areas.ptr, parts);
         PM_LAUNCH_CHECK();
     }
     if (sah) {
-        if (!balanced) {
-            lower_prep_kernel<<<grid_for(nlf, BS, graph ? 4096 : INT_MAX), BS, 0, s>>>(NP, ctx->leaf_ids.ptr, L,
-                                                                                       sc.areas.ptr);
-            PM_LAUNCH_CHECK();
-        }
-        if (!graph) sc.prims_part.reserve(PRIM_SLOTS, s);
-        plan_lower_start_kernel<<<1, 64, 0, s>>>(L, sc.prims_part.ptr);
-        PM_LAUNCH_CHECK();
-        long long An = h.nleaf;
+        long long An = h.nleaf, n_nodes = h.nodes_size;
         for (int ll = 0; graph ? ll < caps->lower_levels : An > 0; ++ll) {
             const long long nAn = graph ? caps->lower : An;
             if (!graph) {
                 sc.lower_flag.reserve(An + 1, s); sc.lower_off.reserve(An + 1, s); sc.lower_list.reserve(An + 1, s);
                 sc.lower_sets.reserve(2 * (size_t)An, s); sc.lower_careas.reserve(2 * (size_t)An, s);
                 seen.lower = std::max(seen.lower, An);
+                nodes.reserve((size_t)(n_nodes + 2 * An), s, (size_t)n_nodes);   // every node split
             }
             NP = node_ptrs(ctx);
             if (balanced)
@@ -2510,7 +2563,8 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
                     NP, ctx->leaf_ids.ptr, L, sc.prim_min.ptr, sc.prim_max.ptr, prm.traversal_cost, LS,
                     sc.lower_flag.ptr, sc.lower_sets.ptr, sc.lower_careas.ptr);
             else {
-                sah_screen_kernel<<<grid_for((nAn + 63) / 64, WPB, graph ? 1024 : INT_MAX), WPB * 64, 0, s>>>(
+                const int npw = screen_nodes(nAn);
+                sah_screen_kernel<<<grid_for((nAn + npw - 1) / npw, WPB, graph ? 1024 : INT_MAX), WPB * 64, 0, s>>>(
                     NP, ctx->leaf_ids.ptr, L, sc.areas.ptr, prm.traversal_cost, prm.sah_leaf_max,
                     prm.sah_empty_bonus, sc.lower_flag.ptr, sc.lower_list.ptr, sc.prims_part.ptr);
                 PM_LAUNCH_CHECK();
@@ -2521,26 +2575,28 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
                     sc.lower_sets.ptr, sc.lower_careas.ptr);
             }
             PM_LAUNCH_CHECK();
-            scan_exclusive(sc.lower_flag.ptr, sc.lower_off.ptr, (int)nAn, sc, s, graph ? &L->An : nullptr);
             const unsigned lseq = mirror ? sc.mirror.take_seq() : 0u;
-            plan_lower_kernel<<<1, 64, 0, s>>>(L, sc.lower_off.ptr, sc.prims_part.ptr,
-                                               mirror ? sc.mirror.dev : nullptr, lseq);
+            LvlMirror::Rec *const mir = mirror ? sc.mirror.dev : nullptr;
+            if (nAn <= PLAN_SCAN) {
+                plan_lower_kernel<true><<<1, PLAN_T, 0, s>>>(L, sc.lower_flag.ptr, sc.lower_off.ptr,
+                                                             sc.prims_part.ptr, mir, lseq);
+            } else {
+                scan_exclusive(sc.lower_flag.ptr, sc.lower_off.ptr, (int)nAn, sc, s, graph ? &L->An : nullptr);
+                plan_lower_kernel<false><<<1, 64, 0, s>>>(L, sc.lower_flag.ptr, sc.lower_off.ptr, sc.prims_part.ptr,
+                                                          mir, lseq);
+            }
+            PM_LAUNCH_CHECK();
+            lower_children_kernel<<<grid_for(nAn, BS, graph ? 4096 : INT_MAX), BS, 0, s>>>(
+                NP, ctx->leaf_ids.ptr, L, prm.propagate_aabbs, sc.lower_flag.ptr, sc.lower_off.ptr,
+                sc.lower_sets.ptr, sc.lower_careas.ptr);
             PM_LAUNCH_CHECK();
             if (!graph) {
                 if (mirror) wait_level(sc, h, lseq, s);
                 else read_state(sc, h, s);
                 if (h.status) throw_status(h);
-                if (h.splits == 0) break;
-                nodes.reserve((size_t)h.nodes_size, s, h.nodes_size - 2 * h.splits);
+                An = 2ll * h.splits;
+                n_nodes = h.nodes_size;
             }
-            NP = node_ptrs(ctx);
-            lower_children_kernel<<<grid_for(nAn, BS, graph ? 4096 : INT_MAX), BS, 0, s>>>(
-                NP, ctx->leaf_ids.ptr, L, prm.propagate_aabbs, sc.lower_flag.ptr, sc.lower_off.ptr,
-                sc.lower_sets.ptr, sc.lower_careas.ptr);
-            PM_LAUNCH_CHECK();
-            plan_lower_advance_kernel<<<1, 64, 0, s>>>(L);
-            PM_LAUNCH_CHECK();
-            if (!graph) An = 2ll * h.splits;
         }
         if (graph) {
             plan_finish_kernel<<<1, 64, 0, s>>>(L, 1);

@@ -113,6 +113,7 @@ struct Lvl {
     int leafTri, nextR, created, child_start, next_active;
     int final_refs, nleaf, level;
     int An, list_base, use_list, splits, lower_base, lower_levels;   // lower levels
+    int ch_An, ch_list_base, ch_use_list;              // the planned lower level, as its children pass reads it
     int cand_n;                                        // lower level: nodes listed for the full SAH search
     int advance;                                       // the children plan is stored, the level not yet advanced
     // a level's active nodes, their first index and segments as the level's
