@@ -23,6 +23,7 @@
 // (TriangleMapBitmapCreator.cu:32-65) is one thread per upper leaf.
 #include <algorithm>
 #include <climits>
+#include <deque>
 #include <type_traits>
 
 #include "pm_device.h"
@@ -2309,7 +2310,7 @@ void read_state(BuildScratch &sc, Lvl &h, hipStream_t s) {
 // seq); the stream is queried now and then, so a pass that failed to run
 // reports the stream's error instead of being waited for
 void wait_level(BuildScratch &sc, Lvl &h, unsigned seq, hipStream_t s) {
-    const LvlMirror::Rec *m = sc.mirror.host;
+    const LvlMirror::Rec *m = sc.mirror.host + (seq & 1u);
     int words[LvlMirror::NW];
     // every word of the record tagged with seq (word 0 is the cheap spin)
     auto take = [&]() {
@@ -2354,6 +2355,47 @@ inline int grid_for(long long n, int per, int cap) {
     return std::max(1, (int)std::min<long long>(blocks_for(std::max(n, 1ll), per), cap));
 }
 
+// refs of a level up to which an eager build launches one level ahead of the
+// state it has taken (the ahead level's buffers are reserved for twice its
+// bound)
+constexpr long long AHEAD_REFS = 1 << 17;
+constexpr long long AHEAD_NODES = 1 << 14;   // the same for the nodes of a lower level
+
+// the sizes of a level (exact, or bounds of them): active nodes, refs,
+// segments, and the nodes, leaf refs and leaf ids written before it
+struct LevelSizes {
+    long long A, R, S, nodes, fin, nleaf;
+    // bounds of the next level's
+    LevelSizes next_bound(int seg) const {
+        return {2 * A, 2 * R, 2 * A + (2 * R + seg - 1) / seg, nodes + 14 * A, fin + 2 * R, nleaf + 2 * A};
+    }
+};
+
+// First sizes of a build's buffers from its triangle count (what the levels'
+// bounds reach on scenes whose refs grow two- to threefold), so that a
+// context's first build does not grow them level by level: every growth is an
+// allocation, a copy and a wait (a context's first build of 1,000,002
+// triangles 11.1 -> 2.7 ms, of 256 meshes with 10.3M 28.9 -> 14.3 ms).  Larger
+// needs still grow.
+void reserve_first(pm_ctx *ctx, int N, int M, int seg, hipStream_t s) {
+    BuildScratch &sc = ctx->scratch;
+    const long long n = N, r = (n <= AHEAD_REFS ? 8 : 5) * n, a = n / 8 + 2ll * M;
+    for (int q = 0; q < 2; ++q) {
+        sc.ref_min[q].reserve((size_t)r + 1, s);
+        sc.ref_max[q].reserve((size_t)r + 1, s);
+        sc.keys[q].reserve((size_t)std::max(12 * a, key_words_host(2 * JOIN_TEST_NODES, true)) + 6, s);
+        sc.node_segbase[q].reserve((size_t)(2 * a) + 2, s);
+        for (DevBuf<int> *b : {&sc.seg_node[q], &sc.seg_start[q], &sc.seg_count[q]})
+            b->reserve((size_t)(2 * a + r / seg) + 1, s);
+    }
+    for (DevBuf<int> *b : {&sc.segL, &sc.segR, &sc.segLoff, &sc.segRoff}) b->reserve((size_t)(a + r / seg) + 1, s);
+    sc.node_lna.reserve((size_t)a + 1, s); sc.node_lref.reserve((size_t)a + 1, s);
+    sc.node_lseg.reserve((size_t)a + 1, s); sc.node_sz.reserve((size_t)a + 1, s);
+    sc.prim_min.reserve((size_t)r + 1, s); sc.prim_max.reserve((size_t)r + 1, s);
+    ctx->leaf_ids.reserve((size_t)n / 2 + 2 * M, s);
+    ctx->nodes.reserve((size_t)(n + n / 2) + 1024 + 16 * M, s, 0);
+}
+
 // The build's kernel sequence.  caps == nullptr: eager (each upper level's
 // leaf pass publishes the level state to the host, each lower level's state is
 // read back; they size the next level's buffers and grids; ends when no node
@@ -2388,10 +2430,14 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
 
     sc.lvl.reserve(1, s);
     const bool mirror = !graph && sc.mirror.ensure();
+    // (a captured batch keeps its buffers: no level reserves more than it needs)
+    const bool run_ahead = mirror && !ctx->graph_exec;
     Lvl *L = sc.lvl.ptr;
     auto tiles = [](long long n, long long per) { return std::max(1ll, (n + per - 1) / per); };
     const int nlb = (int)(8 * tiles(M, NT) + 8);
     if (!graph) {
+        // before the first launch: what grows here loses its contents
+        if (ctx->last_ntris < 0 && !ctx->graph_exec) reserve_first(ctx, N, M, seg, s);
         nodes.reserve(std::max(1024, 2 * M), s, 0);
         sc.ref_min[0].reserve((size_t)N + 1, s); sc.ref_max[0].reserve((size_t)N + 1, s);
         sc.tri_rec.reserve(3 * (size_t)N + 3, s);
@@ -2433,7 +2479,7 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
 
     // the roots' segment table (parity 0); eager: sized by the bound M +
     // ceil(N / seg) (at most one partial segment per root)
-    long long S_now = graph ? caps->segs : M + (N + seg - 1) / seg;
+    const long long S_now = graph ? caps->segs : M + (N + seg - 1) / seg;
     if (!graph) {
         sc.node_segbase[0].reserve((size_t)M + 1, s);
         for (DevBuf<int> *b : {&sc.seg_node[0], &sc.seg_start[0], &sc.seg_count[0]}) b->reserve(S_now + 1, s);
@@ -2450,27 +2496,38 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
     // 12 empty-space nodes and 2 children per active node, at most 2R refs
     // written, at most one segment per child plus one per chunk of its
     // refs), then waits for the state the level's leaf pass publishes (while
-    // the scatter pass runs) to size the next level.  It ends after the
-    // level that creates no active node.
-    long long A_now = M, R_now = N, nodes_now = M, fin_now = 0, nleaf_now = 0;
-    for (int lvl = 0; graph ? lvl < caps->upper_levels : true; ++lvl) {
+    // the scatter pass runs) to size the next level.  A level of up to
+    // AHEAD_REFS refs takes less time than that round trip and the next
+    // launches, so there the host launches the next level too, sized by those
+    // bounds, before it takes the level's state (a 5,316-triangle room with 18
+    // upper and 8 lower levels 833 -> 723 us; 65,002 triangles, whose levels
+    // take longer, 650 -> 637).  The build ends after the level that creates no active node; a
+    // level launched past it has no nodes and writes none.
+    LevelSizes known{M, N, S_now, M, 0, 0};   // the level after the last one whose state is known
+    std::deque<unsigned> out;                 // levels launched after that, not taken yet
+    bool done = false;
+    for (int lvl = 0; graph ? lvl < caps->upper_levels : !done; ++lvl) {
         const int par = lvl & 1, nxt = par ^ 1;
-        const long long A_g = graph ? caps->active : A_now, S_g = graph ? caps->segs : S_now;
+        LevelSizes b = known;
+        for (size_t k = 0; k < out.size(); ++k) b = b.next_bound(seg);
+        const long long A_now = b.A;
+        const long long A_g = graph ? caps->active : A_now, S_g = graph ? caps->segs : b.S;
         if (!graph) {
-            for (DevBuf<int> *b : {&sc.segL, &sc.segR, &sc.segLoff, &sc.segRoff}) b->reserve(S_now + 1, s);
+            for (DevBuf<int> *q : {&sc.segL, &sc.segR, &sc.segLoff, &sc.segRoff}) q->reserve(b.S + 1, s);
             sc.node_lna.reserve(A_now + 1, s); sc.node_lref.reserve(A_now + 1, s); sc.node_lseg.reserve(A_now + 1, s);
             sc.node_sz.reserve(A_now + 1, s);
-            nodes.reserve((size_t)(nodes_now + 14 * A_now + 1), s, (size_t)nodes_now);
-            sc.keys[nxt].reserve((size_t)key_words_host(2 * A_now, A_now < JOIN_TEST_NODES) + 6, s);
-            sc.node_segbase[nxt].reserve(2 * (size_t)A_now + 2, s);
-            sc.lb_words[nxt].reserve(8 * tiles(2 * A_now, NT) + 8, s);
-            const size_t R2 = 2 * (size_t)R_now;
-            sc.prim_min.reserve((size_t)fin_now + R2 + 1, s, (size_t)fin_now);
-            sc.prim_max.reserve((size_t)fin_now + R2 + 1, s, (size_t)fin_now);
-            ctx->leaf_ids.reserve((size_t)nleaf_now + 2 * (size_t)A_now + 1, s, (size_t)nleaf_now);
-            sc.ref_min[nxt].reserve(R2 + 1, s); sc.ref_max[nxt].reserve(R2 + 1, s);
-            const size_t S2 = 2 * (size_t)A_now + (R2 + seg - 1) / seg + 1;
-            for (DevBuf<int> *b : {&sc.seg_node[nxt], &sc.seg_start[nxt], &sc.seg_count[nxt]}) b->reserve(S2, s);
+            const LevelSizes w = b.next_bound(seg);   // what the level may write
+            nodes.reserve((size_t)w.nodes + 1, s, (size_t)b.nodes);
+            // (replicated if the level turns out to have few nodes)
+            sc.keys[nxt].reserve((size_t)std::max(key_words_host(w.A, false),
+                                                  key_words_host(std::min(w.A, 2ll * JOIN_TEST_NODES), true)) + 6, s);
+            sc.node_segbase[nxt].reserve((size_t)w.A + 2, s);
+            sc.lb_words[nxt].reserve(8 * tiles(w.A, NT) + 8, s);
+            sc.prim_min.reserve((size_t)w.fin + 1, s, (size_t)b.fin);
+            sc.prim_max.reserve((size_t)w.fin + 1, s, (size_t)b.fin);
+            ctx->leaf_ids.reserve((size_t)w.nleaf + 1, s, (size_t)b.nleaf);
+            sc.ref_min[nxt].reserve((size_t)w.R + 1, s); sc.ref_max[nxt].reserve((size_t)w.R + 1, s);
+            for (DevBuf<int> *q : {&sc.seg_node[nxt], &sc.seg_start[nxt], &sc.seg_count[nxt]}) q->reserve(w.S + 1, s);
         }
         const LevelBufs B = level_bufs(par);
         const NodePtrs NP = node_ptrs(ctx);
@@ -2486,7 +2543,7 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
         const unsigned seq = mirror ? sc.mirror.take_seq() : 0u;
         leaf_pass_kernel<<<graph ? std::min(g3, 2048) : g3, LBS, 0, s>>>(
             NP, L, B, par, LS, seg, sc.keys[par].ptr, sc.keys[nxt].ptr, prm.empty_space_splitting,
-            prm.empty_space_threshold, mirror ? sc.mirror.dev : nullptr, seq);
+            prm.empty_space_threshold, mirror ? sc.mirror.dev + (seq & 1u) : nullptr, seq);
         PM_LAUNCH_CHECK();
         const int g4 = std::max(grid_for(S_g, WPB, INT_MAX), grid_for(A_g, BS, INT_MAX));
         launch_scatter_pass(seg, div, graph ? std::min(g4, 2048) : g4, s, NP, (const Lvl *)L, B, LS, seg,
@@ -2494,21 +2551,25 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
                             (const float4 *)sc.ref_max[par].ptr, sc.ref_min[nxt].ptr, sc.ref_max[nxt].ptr,
                             sc.prim_min.ptr, sc.prim_max.ptr, sc.keys[nxt].ptr, ctx->leaf_ids.ptr, dg);
         PM_LAUNCH_CHECK();
-        if (!graph) {
-            if (mirror) wait_level(sc, h, seq, s);
+        if (graph) continue;
+        out.push_back(seq);
+        const size_t ahead = run_ahead && known.R <= AHEAD_REFS ? 1 : 0;
+        while (out.size() > ahead && !done) {
+            const int taken = (lvl + 1 - (int)out.size()) & 1;   // the taken level's parity
+            if (mirror) wait_level(sc, h, out.front(), s);
             else read_state(sc, h, s);
+            out.pop_front();
             if (h.status) throw_status(h);
             ctx->level_refs.push_back(h.R);
             seen.refs = std::max<long long>(seen.refs, h.R);
             seen.active = std::max<long long>(seen.active, h.A);
             seen.segs = std::max<long long>(seen.segs, h.S);
-            seen.segs = std::max<long long>(seen.segs, h.scanS[nxt]);
-            if (h.created == 0) break;
+            seen.segs = std::max<long long>(seen.segs, h.scanS[taken ^ 1]);
+            done = h.created == 0;
             // the next level as the advance will make it
             Lvl n = h;
             advance_level(&n);
-            A_now = n.A; R_now = n.R; S_now = h.scanS[nxt];
-            nodes_now = n.nodes_size; fin_now = n.final_refs; nleaf_now = n.nleaf;
+            known = LevelSizes{n.A, n.R, h.scanS[taken ^ 1], n.nodes_size, n.final_refs, n.nleaf};
         }
     }
     // the last level's advance
@@ -2548,13 +2609,17 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
         PM_LAUNCH_CHECK();
     }
     if (sah) {
-        long long An = h.nleaf, n_nodes = h.nodes_size;
-        for (int ll = 0; graph ? ll < caps->lower_levels : An > 0; ++ll) {
+        // as the upper levels, a small level's successor (at most two children
+        // a node) is launched before its state is taken
+        long long known_An = h.nleaf, known_nodes = h.nodes_size;
+        out.clear();
+        for (int ll = 0; graph ? ll < caps->lower_levels : known_An > 0; ++ll) {
+            const long long An = known_An << out.size();
+            const long long n_nodes = known_nodes + (out.empty() ? 0 : 2 * known_An);
             const long long nAn = graph ? caps->lower : An;
             if (!graph) {
                 sc.lower_flag.reserve(An + 1, s); sc.lower_off.reserve(An + 1, s); sc.lower_list.reserve(An + 1, s);
                 sc.lower_sets.reserve(2 * (size_t)An, s); sc.lower_careas.reserve(2 * (size_t)An, s);
-                seen.lower = std::max(seen.lower, An);
                 nodes.reserve((size_t)(n_nodes + 2 * An), s, (size_t)n_nodes);   // every node split
             }
             NP = node_ptrs(ctx);
@@ -2576,7 +2641,7 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
             }
             PM_LAUNCH_CHECK();
             const unsigned lseq = mirror ? sc.mirror.take_seq() : 0u;
-            LvlMirror::Rec *const mir = mirror ? sc.mirror.dev : nullptr;
+            LvlMirror::Rec *const mir = mirror ? sc.mirror.dev + (lseq & 1u) : nullptr;
             if (nAn <= PLAN_SCAN) {
                 plan_lower_kernel<true><<<1, PLAN_T, 0, s>>>(L, sc.lower_flag.ptr, sc.lower_off.ptr,
                                                              sc.prims_part.ptr, mir, lseq);
@@ -2590,12 +2655,17 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
                 NP, ctx->leaf_ids.ptr, L, prm.propagate_aabbs, sc.lower_flag.ptr, sc.lower_off.ptr,
                 sc.lower_sets.ptr, sc.lower_careas.ptr);
             PM_LAUNCH_CHECK();
-            if (!graph) {
-                if (mirror) wait_level(sc, h, lseq, s);
+            if (graph) continue;
+            out.push_back(lseq);
+            const size_t ahead = run_ahead && known_An <= AHEAD_NODES ? 1 : 0;
+            while (out.size() > ahead && known_An > 0) {
+                if (mirror) wait_level(sc, h, out.front(), s);
                 else read_state(sc, h, s);
+                out.pop_front();
                 if (h.status) throw_status(h);
-                An = 2ll * h.splits;
-                n_nodes = h.nodes_size;
+                seen.lower = std::max(seen.lower, known_An);
+                known_An = 2ll * h.splits;
+                known_nodes = h.nodes_size;
             }
         }
         if (graph) {

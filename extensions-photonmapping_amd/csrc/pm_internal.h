@@ -150,12 +150,14 @@ struct LvlMirror {
     struct Rec {
         unsigned long long w[NW];
     };
-    Rec *host = nullptr;   // coherent, mapped
-    Rec *dev = nullptr;    // the device's address of it
+    Rec *host = nullptr;   // coherent, mapped: two records, a level's is [number & 1]
+    Rec *dev = nullptr;    // the device's address of them
     unsigned next_seq = 0;
-    // the next level's number: never 0, the tag of a record no level wrote
+    // the next level's number: odd and even in turn (a level launched before
+    // the one before it is taken writes the other record), never 0, the tag
+    // of a record no level wrote
     unsigned take_seq() {
-        if (++next_seq == 0u) next_seq = 1u;
+        if (++next_seq == 0u) next_seq = 2u;
         return next_seq;
     }
     ~LvlMirror() { if (host) (void)hipHostFree(host); }
@@ -170,7 +172,7 @@ struct LvlMirror {
             failed = true;
             return false;
         }
-        if (hipHostMalloc((void **)&host, sizeof(Rec), hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess ||
+        if (hipHostMalloc((void **)&host, 2 * sizeof(Rec), hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess ||
             hipHostGetDevicePointer((void **)&dev, host, 0) != hipSuccess) {
             (void)hipGetLastError();
             if (host) (void)hipHostFree(host);
@@ -179,7 +181,7 @@ struct LvlMirror {
             failed = true;
             return false;
         }
-        for (int t = 0; t < NW; ++t) __atomic_store_n(&host->w[t], 0ull, __ATOMIC_RELEASE);
+        for (int t = 0; t < 2 * NW; ++t) __atomic_store_n(&host[t / NW].w[t % NW], 0ull, __ATOMIC_RELEASE);
         return true;
     }
 };
