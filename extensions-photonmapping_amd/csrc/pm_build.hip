@@ -1404,12 +1404,6 @@ __host__ __device__ void advance_level(Lvl *L) {
     if (L->A > 0 && L->level >= L->max_levels) lvl_fail(L, PM_ERR_DEPTH);
 }
 
-// ExtractIndexFromAabb (TriangleUpper.h:43-52)
-__global__ void extract_index_kernel(const float4 *__restrict__ fmin, int *__restrict__ out, const Lvl *__restrict__ L) {
-    const int n = L->status ? 0 : L->final_refs;
-    GRID_STRIDE(i, n) out[i] = __float_as_int(fmin[i].w);
-}
-
 // PropagateParentAabb<true> (EmptySpaceSplitting.h:333-368)
 __global__ void propagate_parent_kernel(NodePtrs N, const int *__restrict__ leaf_ids, const Lvl *__restrict__ L) {
     const int n = L->status ? 0 : L->nleaf;
@@ -2265,24 +2259,30 @@ void scan_exclusive2(const int *in0, int *out0, const int *in1, int *out1, int n
 
 namespace {
 
-__global__ void single_offsets_kernel(int *off, int N) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) { off[0] = 0; off[1] = N; }
-}
-
 // a build's first launch, each part over the whole grid: the level state;
 // one root per mesh (TriangleMapUpperCreator.cu:128-137): root m covers
 // triangles [off[m], off[m+1]) and is its own parent; the roots' box keys
 // (AabbMemset, ReduceSegments.h:328-336); the look-back words and tickets of
 // the roots' segment scan (parity 1) and of the first level's leaf pass
-// (parity 0)
-__global__ void build_init_kernel(Lvl *L, Lvl v, NodePtrs N, const int *__restrict__ off, int M, int *keys,
-                                  int repl, unsigned long long *lb0, unsigned long long *lb1, int nlb, int *ctr) {
+// (parity 0).  A single mesh of ntris triangles (M == 1, off unused) needs no
+// scan: its S segments follow from ntris and are written here too.
+__global__ void build_init_kernel(Lvl *L, Lvl v, NodePtrs N, const int *__restrict__ off, int M, int ntris, int *keys,
+                                  int repl, unsigned long long *lb0, unsigned long long *lb1, int nlb, int *ctr,
+                                  int *__restrict__ segbase, int *__restrict__ sn, int *__restrict__ ss,
+                                  int *__restrict__ sc, int S, int seg) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *L = v;
     GRID_STRIDE(m, M) {
         zero_node(N, m);
-        N.prim_index[m] = off[m];
-        N.bitmap[m] = off[m + 1] - off[m];
+        N.prim_index[m] = M > 1 ? off[m] : 0;
+        N.bitmap[m] = M > 1 ? off[m + 1] - off[m] : ntris;
         N.parent[m] = m;
+    }
+    if (M == 1) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            segbase[0] = 0;
+            segbase[1] = S;
+        }
+        GRID_STRIDE(k, S) write_segment(sn, ss, sc, k, 0, 0, ntris, seg, k);
     }
     key_reset(keys, M, repl);
     GRID_STRIDE(k, nlb) {
@@ -2445,12 +2445,24 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
         sc.lb_ctr.reserve(4, s);
         for (int q = 0; q < 2; ++q) sc.lb_words[q].reserve(nlb, s);
     }
+    // the roots' segment table (parity 0); eager: sized by the bound M +
+    // ceil(N / seg) (at most one partial segment per root)
+    const long long S_now = graph ? caps->segs : M + (N + seg - 1) / seg;
+    if (!graph) {
+        sc.node_segbase[0].reserve((size_t)M + 1, s);
+        for (DevBuf<int> *b : {&sc.seg_node[0], &sc.seg_start[0], &sc.seg_count[0]}) b->reserve(S_now + 1, s);
+    }
+    const int S1 = M == 1 ? (N + seg - 1) / seg : 0;   // a single root's segments
+    h.scanS[0] = S1;
+    if (S1 > h.cap_segs) lvl_fail(&h, PM_ERR_CAPACITY);
     {
-        const long long g = std::max({(long long)blocks_for(M, BS),
+        const long long g = std::max({(long long)blocks_for(M, BS), (long long)grid_for(S1, BS, 64),
                                       (long long)grid_for(6ll * M * (repl0 ? KEY_REPL : 1), BS, 1024),
                                       (long long)grid_for(nlb, BS, 64)});
-        build_init_kernel<<<(int)g, BS, 0, s>>>(L, h, node_ptrs(ctx), off_dev, M, sc.keys[0].ptr, repl0,
-                                                 sc.lb_words[0].ptr, sc.lb_words[1].ptr, nlb, sc.lb_ctr.ptr);
+        build_init_kernel<<<(int)g, BS, 0, s>>>(L, h, node_ptrs(ctx), off_dev, M, N, sc.keys[0].ptr, repl0,
+                                                 sc.lb_words[0].ptr, sc.lb_words[1].ptr, nlb, sc.lb_ctr.ptr,
+                                                 sc.node_segbase[0].ptr, sc.seg_node[0].ptr, sc.seg_start[0].ptr,
+                                                 sc.seg_count[0].ptr, h.status ? 0 : S1, seg);
         PM_LAUNCH_CHECK();
     }
     if (N > 0) {
@@ -2477,18 +2489,13 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
         return B;
     };
 
-    // the roots' segment table (parity 0); eager: sized by the bound M +
-    // ceil(N / seg) (at most one partial segment per root)
-    const long long S_now = graph ? caps->segs : M + (N + seg - 1) / seg;
-    if (!graph) {
-        sc.node_segbase[0].reserve((size_t)M + 1, s);
-        for (DevBuf<int> *b : {&sc.seg_node[0], &sc.seg_start[0], &sc.seg_count[0]}) b->reserve(S_now + 1, s);
+    if (M > 1) {
+        root_segments_kernel<<<(int)tiles(M, NT), LBS, 0, s>>>(node_ptrs(ctx), L, sc.node_segbase[0].ptr,
+                                                               sc.seg_node[0].ptr, sc.seg_start[0].ptr,
+                                                               sc.seg_count[0].ptr, sc.lb_words[1].ptr,
+                                                               sc.lb_ctr.ptr + 1, M, seg);
+        PM_LAUNCH_CHECK();
     }
-    root_segments_kernel<<<(int)tiles(M, NT), LBS, 0, s>>>(node_ptrs(ctx), L, sc.node_segbase[0].ptr,
-                                                           sc.seg_node[0].ptr, sc.seg_start[0].ptr,
-                                                           sc.seg_count[0].ptr, sc.lb_words[1].ptr,
-                                                           sc.lb_ctr.ptr + 1, M, seg);
-    PM_LAUNCH_CHECK();
 
     // A level is three launches (classify, leaf and scatter passes; see the
     // level kernels above), launched back to back.  The eager build reserves
@@ -2582,9 +2589,6 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
     const long long nref = graph ? caps->leaf_refs : h.final_refs;
     const long long nlf = graph ? caps->leaf_ids : h.nleaf;
     if (!graph) ctx->prim_indices.reserve((size_t)h.final_refs + 1, s);
-    extract_index_kernel<<<grid_for(nref, BS, graph ? 8192 : INT_MAX), BS, 0, s>>>(sc.prim_min.ptr,
-                                                                                    ctx->prim_indices.ptr, L);
-    PM_LAUNCH_CHECK();
     if (!prm.empty_space_splitting && prm.propagate_aabbs) {
         propagate_parent_kernel<<<grid_for(nlf, BS, graph ? 4096 : INT_MAX), BS, 0, s>>>(NP, ctx->leaf_ids.ptr, L);
         PM_LAUNCH_CHECK();
@@ -2593,8 +2597,7 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
     const bool sah = prm.lower_algorithm != PM_LOWER_BITMAP;   // SAH or balanced: lower levels
     const bool need_areas = prm.lower_algorithm == PM_LOWER_SAH;
     if (need_areas && !graph) sc.areas.reserve((size_t)h.final_refs + 1, s);
-    build_leaf_view(ctx, need_areas ? sc.areas.ptr : nullptr, false, s, graph ? &L->final_refs : nullptr,
-                    N > 0 ? sc.tri_rec.ptr : nullptr);
+    build_leaf_slots(ctx, sc.prim_min.ptr, sc.tri_rec.ptr, need_areas ? sc.areas.ptr : nullptr, L, s);
 
     // lower stage
     const bool balanced = prm.lower_algorithm == PM_LOWER_BALANCED;
@@ -2709,10 +2712,7 @@ void upload_offsets(pm_ctx *ctx, const int *mesh_offsets, int N, int M, hipStrea
         if (off_h[m] > off_h[m + 1]) throw Error{PM_ERR_ARG, "mesh offsets must be non-decreasing"};
     if (off_h[0] != 0 || off_h[M] != N) throw Error{PM_ERR_ARG, "mesh offsets must span [0, n]"};
     sc.mesh_off.reserve((size_t)M + 1, s);
-    if (M == 1) {   // {0, N}: written on the device, no staged copy and no stream wait
-        single_offsets_kernel<<<1, 64, 0, s>>>(sc.mesh_off.ptr, N);
-        PM_LAUNCH_CHECK();
-    } else {
+    if (M > 1) {   // (a single mesh's {0, N} is never read: no copy and no stream wait)
         PM_HIP(hipMemcpyAsync(sc.mesh_off.ptr, off_h.data(), (M + 1) * sizeof(int), hipMemcpyHostToDevice, s));
         PM_HIP(hipStreamSynchronize(s));
     }

@@ -293,15 +293,13 @@ int sync_graph_state(pm_ctx *ctx, hipStream_t s);
 void destroy_graph(pm_ctx *ctx);
 // pm_trace.hip
 void build_trace_view(pm_ctx *ctx, hipStream_t s);
-// the two halves of the trace view: packed nodes, and the leaf slots'
-// triangles (plus their areas when `areas` is given; `check` verifies the
-// prim indices, needed for uploaded trees only).  With n_dev / m_dev the
-// count is read on the device and ctx's count is its upper bound.  `rec`:
-// the triangles' leaf records in triangle order (3 float4 each), copied
-// instead of formed from the vertex arrays.
+// the two halves of a build's trace view.  Nodes: packed nodes and leaf records
+// (n_dev: the count on the device, ctx's is its upper bound).  Leaf slots: prim
+// indices, leaf triangles and (areas not null) areas of the final refs, from the
+// triangles' leaf records `rec` (3 float4 each); the count is L's, ctx's its
+// upper bound.
 void build_node_view(pm_ctx *ctx, hipStream_t s, const int *n_dev = nullptr);
-void build_leaf_view(pm_ctx *ctx, float *areas, bool check, hipStream_t s, const int *m_dev = nullptr,
-                     const float4 *rec = nullptr);
+void build_leaf_slots(pm_ctx *ctx, const float4 *refs, const float4 *rec, float *areas, const Lvl *L, hipStream_t s);
 void trace_canvas(pm_ctx *ctx, int algo, const float4 *org, const float4 *dir, int nrays, const float4 *n0,
                   const float4 *n1, const float4 *n2, const uchar4 *c0, const pm_light &light, int max_bounces,
                   uchar4 *canvas, const pm_trace_params &prm, hipStream_t s);
