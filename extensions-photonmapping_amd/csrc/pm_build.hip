@@ -416,16 +416,12 @@ __device__ __forceinline__ int wave_count() { return (gridDim.x * blockDim.x) >>
 
 // EmptySpaceSplitting2 (EmptySpaceSplitting.h:74-184): a chain of split
 // nodes with empty leaves between the node and its parent.
-__device__ __forceinline__ void empty_chain_node_at(const NodePtrs &N, int i, int A, int active_index, int pl,
-                                                    int eaddr_i) {
-    const int leafID = active_index + i;
-    const int start = active_index + A + eaddr_i;
+__device__ __forceinline__ void empty_chain_node_at(const NodePtrs &N, int leafID, int start, int pl, int parentID,
+                                                    bool is_left, f3 minP, f3 maxP) {
     const int cnt = 2 * __popc(pl);
     for (int j = 0; j < cnt; ++j) zero_node(N, start + j);
-    const int parentID = N.parent[leafID];
-    if (N.children[parentID].x == leafID) N.children[parentID].x = start;
+    if (is_left) N.children[parentID].x = start;
     else N.children[parentID].y = start;
-    const f3 minP = mk3(N.bmin[leafID]), maxP = mk3(N.bmax[leafID]);
     int pid = start;
     for (int a = 0; a < 3; ++a) {
         if (!(pl & (1 << a))) continue;
@@ -621,18 +617,24 @@ __device__ __forceinline__ void block_scan(const int *v, int *pre, int *tot, int
     __syncthreads();
 }
 
-// the device buffers the three level passes share
+// The device buffers the three level passes share.  What a pass reads of a
+// segment or of a node is one record, so that it waits for it once: at every
+// level a pass is a chain of dependent loads (0.7 us each across the launches'
+// cache boundary), and on small levels that chain is all it takes.
 struct LevelBufs {
-    const int *segbase;                           // per active node: first segment; A + 1 entries
-    const int *seg_node, *seg_start, *seg_count;  // the level's segment table
-    int *segL, *segR;                             // per segment: refs on each side (classify pass)
-    int *segLoff, *segRoff;                       // per segment: refs on each side before it, S + 1 entries
-    int2 *lna, *lref, *lseg;                      // per active node: leaf slots / leaf refs / next-level
-                                                  // segments of non-leaf children before it (left, right)
-    int4 *nsz;                                    // per active node: children sizes, side offsets of its first segment
-    int *segbase_n, *seg_node_n, *seg_start_n, *seg_count_n;   // the same for the next level
-    unsigned long long *lb, *lb_n;                // look-back words of this level's leaf pass and the next's
-    int *ctr;                                     // leaf pass tickets by level parity
+    const int *segbase;        // per active node: first segment; A + 1 entries
+    const int4 *seg;           // the level's segment table: {node, first ref, count, k: the node's k-th}
+    int seg_last;              // the table's last entry (a wave reads its first record before it knows S)
+    int *segL, *segR;          // per segment: refs on each side (classify pass)
+    int *segLoff, *segRoff;    // per segment: refs on each side before it, S + 1 entries
+    int4 *rec;                 // per active node, 3 records (leaf pass to scatter pass):
+                               //   children sizes (left, right), side offsets of its first segment
+                               //   leaf slots before it (left, right), leaf refs before it
+                               //   next-level segments of non-leaf children before it, split axis, plane bits
+    int *segbase_n;            // the same for the next level
+    int4 *seg_n;
+    unsigned long long *lb, *lb_n;   // look-back words of this level's leaf pass and the next's
+    int *ctr;                  // leaf pass tickets by level parity
 };
 
 // what prepare_node reads of active node i: its six box keys and (empty-space
@@ -640,6 +642,7 @@ struct LevelBufs {
 struct NodeIn {
     int2 k01, k23, k45;
     float4 pmn, pmx;
+    int parent;
 };
 
 __device__ __forceinline__ void load_node(const NodePtrs &N, int i, int node, const int *__restrict__ keys,
@@ -655,6 +658,7 @@ __device__ __forceinline__ void load_node(const NodePtrs &N, int i, int node, co
     if (empty_space) {
         v.pmn = N.bmin[node];
         v.pmx = N.bmax[node];
+        v.parent = N.parent[node];
     }
 }
 
@@ -674,9 +678,9 @@ __device__ __forceinline__ void node_split(f3 rMin, f3 rMax, int &ax, float &sp)
 // ReduceAabb result -> node box, CalcEmptySpaceSplits (EmptySpaceSplitting.h:
 // 10-70) and the split plane for an active node, from what load_node read
 __device__ __forceinline__ void prepare_node(const NodePtrs &N, int node, const NodeIn &v, bool empty_space,
-                                             float thr, int &pl) {
-    const f3 rMin = {unkey(v.k01.x), unkey(v.k01.y), unkey(v.k23.x)};
-    const f3 rMax = {unkey(v.k23.y), unkey(v.k45.x), unkey(v.k45.y)};
+                                             float thr, int &pl, int &ax, float &sp, f3 &rMin, f3 &rMax) {
+    rMin = {unkey(v.k01.x), unkey(v.k01.y), unkey(v.k23.x)};
+    rMax = {unkey(v.k23.y), unkey(v.k45.x), unkey(v.k45.y)};
     pl = 0;
     if (empty_space) {
         const f3 pMin = mk3(v.pmn), pMax = mk3(v.pmx);
@@ -689,8 +693,6 @@ __device__ __forceinline__ void prepare_node(const NodePtrs &N, int node, const 
     }
     N.bmin[node] = make_float4(rMin.x, rMin.y, rMin.z, 0.0f);
     N.bmax[node] = make_float4(rMax.x, rMax.y, rMax.z, 0.0f);
-    int ax;
-    float sp;
     node_split(rMin, rMax, ax, sp);
     N.split[node] = sp;
     N.info[node] = (int8_t)ax;
@@ -698,11 +700,9 @@ __device__ __forceinline__ void prepare_node(const NodePtrs &N, int node, const 
 
 // the segment table entry of a node's k-th segment (Segment,
 // TriangleMapUpperCreator.cu:207-239)
-__device__ __forceinline__ void write_segment(int *__restrict__ sn, int *__restrict__ ss, int *__restrict__ sc,
-                                              int sg, int i, int first_ref, int count, int seg, int k) {
-    sn[sg] = i;
-    ss[sg] = first_ref + k * seg;
-    sc[sg] = min(seg, count - k * seg);
+__device__ __forceinline__ void write_segment(int4 *__restrict__ table, int sg, int i, int first_ref, int count,
+                                              int seg, int k) {
+    table[sg] = make_int4(i, first_ref + k * seg, min(seg, count - k * seg), k);
 }
 
 // segments a root's own thread writes; the rest of a long root's segments are
@@ -713,8 +713,7 @@ constexpr int SEG_DIRECT = 4;
 // look-back scan of the roots' segment counts.  Uses the look-back words and
 // ticket of level parity 1 (level 0's leaf pass clears them for level 1).
 __global__ __launch_bounds__(LBS) void root_segments_kernel(NodePtrs N, Lvl *L, int *__restrict__ segbase,
-                                                           int *__restrict__ sn, int *__restrict__ ss,
-                                                           int *__restrict__ sc, unsigned long long *lbw, int *ctr,
+                                                           int4 *__restrict__ table, unsigned long long *lbw, int *ctr,
                                                            int M, int seg) {
     __shared__ int s_tile, s_first;
     __shared__ int s_xpre[NT], s_segpre[NT], s_pi[NT], s_cnt[NT];
@@ -761,7 +760,7 @@ __global__ __launch_bounds__(LBS) void root_segments_kernel(NodePtrs N, Lvl *L, 
                 segbase[i] = eseg + q;
                 if (fits)
                     for (int k = 0; k < min(ns, SEG_DIRECT); ++k)
-                        write_segment(sn, ss, sc, eseg + q + k, i, pi[j], cnt[j], seg, k);
+                        write_segment(table, eseg + q + k, i, pi[j], cnt[j], seg, k);
                 s_xpre[li] = x;
                 s_segpre[li] = q;
                 s_pi[li] = pi[j];
@@ -780,7 +779,7 @@ __global__ __launch_bounds__(LBS) void root_segments_kernel(NodePtrs N, Lvl *L, 
                 if (s_xpre[mid] <= ls) lo = mid; else hi = mid - 1;
             }
             const int k = SEG_DIRECT + ls - s_xpre[lo];
-            write_segment(sn, ss, sc, eseg + s_segpre[lo] + k, i0 + lo, s_pi[lo], s_cnt[lo], seg, k);
+            write_segment(table, eseg + s_segpre[lo] + k, i0 + lo, s_pi[lo], s_cnt[lo], seg, k);
         }
         if (tile == ntiles - 1 && t == 0) {
             const long long S = (long long)eseg + tot[0];
@@ -791,71 +790,38 @@ __global__ __launch_bounds__(LBS) void root_segments_kernel(NodePtrs N, Lvl *L, 
     }
 }
 
-// SetSplitSide (TriangleUpperChildren.h:10-62) for one segment: its counts
-// of refs on the left and on the right of its node's plane
-template <int SEGT, bool DIV>
-__device__ __forceinline__ void classify_segment(int ax, float sp, f3 nmn, f3 nmx, int start, int count,
-                                                 const float4 *__restrict__ rmin, const float4 *__restrict__ rmax,
-                                                 const DivideGeom &dg, int &cl, int &cr) {
-    const int lane = threadIdx.x & 63;
-    cl = 0; cr = 0;
-    // the chunk's iterations (wave-uniform): groups of up to 16 while the
-    // chunk has that many refs left, then groups of 2
-    const int its = (count + 63) >> 6;
-    if (!DIV) {
-        // the split axis' coordinates only, loaded without branches (lanes
-        // past the chunk re-read its first ref) so that a group's loads all
-        // issue before its first compare
-        const float *lo = reinterpret_cast<const float *>(rmin + start) + (ax - AX_X);
-        const float *hi = reinterpret_cast<const float *>(rmax + start) + (ax - AX_X);
-        auto group = [&](int it0, auto G) {
-            float a[G.value], b[G.value];
-#pragma unroll
-            for (int q = 0; q < G.value; ++q) {
-                const int j = (it0 + q) * 64 + lane;
-                const int jj = j < count ? j : 0;
-                a[q] = lo[4 * jj];
-                b[q] = hi[4 * jj];
-            }
-#pragma unroll
-            for (int q = 0; q < G.value; ++q) {
-                const int j = (it0 + q) * 64 + lane;
-                cl += __popcll(__ballot(j < count && a[q] <= sp));
-                cr += __popcll(__ballot(j < count && sp < b[q]));
-            }
-        };
-        constexpr int GB = SEGT / 64 < 16 ? SEGT / 64 : 16;
-        int it = 0;
-        for (; it + GB <= its; it += GB) group(it, std::integral_constant<int, GB>{});
-        for (; it < its; it += 2) group(it, std::integral_constant<int, 2>{});
-    } else {
-        for (int it = 0; it < its; ++it) {
-            const int j = it * 64 + lane;
-            const bool valid = j < count;
-            bool l = false, r = false;
-            if (valid) {
-                const float4 mn = rmin[start + j];
-                l = comp4(mn, ax) <= sp;
-                r = sp < comp4(rmax[start + j], ax);
-                if (l && r) divide_sides(dg, mn.w, ax, sp, nmn, nmx, l, r);
-            }
-            cl += __popcll(__ballot(l));
-            cr += __popcll(__ballot(r));
-        }
-    }
-}
-
-// the level's segments, one wave each; a segment's node's plane comes from
-// the node's box keys (the values the leaf pass gives the node record)
+// SetSplitSide (TriangleUpperChildren.h:10-62): the counts of a segment's refs
+// on the left and on the right of its node's plane, one wave per segment; the
+// plane comes from the node's box keys (the values the leaf pass gives the node
+// record).  A wave's first segment record is loaded with the level's sizes, and
+// a segment's first 128 refs (all of it on the deep levels) with its node's
+// keys: two waits instead of four.
 template <int SEGT, bool DIV>
 __global__ __launch_bounds__(WPB * 64) void classify_pass_kernel(const Lvl *L, LevelBufs B, int par,
                                                                  const int *__restrict__ keys,
                                                                  const float4 *__restrict__ rmin,
                                                                  const float4 *__restrict__ rmax, DivideGeom dg) {
+    const int lane = threadIdx.x & 63;
+    const int s0 = __builtin_amdgcn_readfirstlane(wave_index());
+    int4 r = B.seg[min(s0, B.seg_last)];
     const int S = L->status ? 0 : L->scanS[par];
     const bool repl = L->scanR[par];
-    for (int s = wave_index(); s < S; s += wave_count()) {
-        const int i = __builtin_amdgcn_readfirstlane(B.seg_node[s]);
+    for (int s = s0; s < S; s += wave_count()) {
+        if (s != s0) r = B.seg[s];
+        const int i = __builtin_amdgcn_readfirstlane(r.x), start = __builtin_amdgcn_readfirstlane(r.y);
+        const int count = __builtin_amdgcn_readfirstlane(r.z);
+        // the chunk's iterations (wave-uniform): the first two here, then
+        // groups of up to 16 while the chunk has that many refs left, then of 2
+        const int its = (count + 63) >> 6;
+        constexpr int PRE = 2;
+        float4 mn[PRE], mx[PRE];
+#pragma unroll
+        for (int q = 0; q < PRE; ++q) {
+            const int j = q * 64 + lane;
+            const int k = start + (j < count ? j : 0);
+            mn[q] = rmin[k];
+            mx[q] = rmax[k];
+        }
         int k[6];
         read_keys(keys, i, repl, k);
         const f3 rMin = {unkey(k[0]), unkey(k[1]), unkey(k[2])};
@@ -863,9 +829,49 @@ __global__ __launch_bounds__(WPB * 64) void classify_pass_kernel(const Lvl *L, L
         int ax;
         float sp;
         node_split(rMin, rMax, ax, sp);
-        int cl, cr;
-        classify_segment<SEGT, DIV>(ax, sp, rMin, rMax, B.seg_start[s], B.seg_count[s], rmin, rmax, dg, cl, cr);
-        if ((threadIdx.x & 63) == 0) { B.segL[s] = cl; B.segR[s] = cr; }
+        int cl = 0, cr = 0;
+        auto side = [&](bool valid, const float4 &lo, const float4 &hi) {
+            bool l = valid && comp4(lo, ax) <= sp, rr = valid && sp < comp4(hi, ax);
+            if (DIV && l && rr) divide_sides(dg, lo.w, ax, sp, rMin, rMax, l, rr);
+            cl += __popcll(__ballot(l));
+            cr += __popcll(__ballot(rr));
+        };
+#pragma unroll
+        for (int q = 0; q < PRE; ++q) side(q * 64 + lane < count, mn[q], mx[q]);
+        if (DIV) {
+            for (int it = PRE; it < its; ++it) {
+                const int j = it * 64 + lane;
+                const int at = start + (j < count ? j : 0);
+                side(j < count, rmin[at], rmax[at]);
+            }
+        } else {
+            // the split axis' coordinates only, loaded without branches (lanes
+            // past the chunk re-read its first ref) so that a group's loads all
+            // issue before its first compare
+            const float *lo = reinterpret_cast<const float *>(rmin + start) + (ax - AX_X);
+            const float *hi = reinterpret_cast<const float *>(rmax + start) + (ax - AX_X);
+            auto group = [&](int it0, auto G) {
+                float a[G.value], b[G.value];
+#pragma unroll
+                for (int q = 0; q < G.value; ++q) {
+                    const int j = (it0 + q) * 64 + lane;
+                    const int jj = j < count ? j : 0;
+                    a[q] = lo[4 * jj];
+                    b[q] = hi[4 * jj];
+                }
+#pragma unroll
+                for (int q = 0; q < G.value; ++q) {
+                    const int j = (it0 + q) * 64 + lane;
+                    cl += __popcll(__ballot(j < count && a[q] <= sp));
+                    cr += __popcll(__ballot(j < count && sp < b[q]));
+                }
+            };
+            constexpr int GB = SEGT / 64 < 14 ? SEGT / 64 : 14;
+            int it = PRE;
+            for (; it + GB <= its; it += GB) group(it, std::integral_constant<int, GB>{});
+            for (; it < its; it += 2) group(it, std::integral_constant<int, 2>{});
+        }
+        if (lane == 0) { B.segL[s] = cl; B.segR[s] = cr; }
     }
 }
 
@@ -911,81 +917,95 @@ constexpr int SEG_LDS = 2048;
 // The level's node work and children plan.  par: the level's parity.
 // The blocks read the level's sizes once (scanA/scanAI/scanS[par]), with
 // their first ticket; the last tile writes the next level's into [par ^ 1].
+// The last tile plans on a copy of the level state in LDS, loaded with its
+// nodes (nothing else writes the state in this pass but a failed look-back its
+// status, which is looked at again), and stores and publishes it from there; a
+// node's parent and its side are loaded before the look-back, not after it.
 __global__ __launch_bounds__(LBS) void leaf_pass_kernel(NodePtrs N, Lvl *L, LevelBufs B, int par, int LS, int seg,
                                                        const int *__restrict__ keys, int *__restrict__ keys_next,
                                                        int empty_space, float thr, LvlMirror::Rec *mirror,
                                                        unsigned seq) {
+    static_assert(NPT == 1, "one node per thread");
     __shared__ int s_tile;
     __shared__ int s_w[7][LBS / 64];
     __shared__ long long s_ex[8];
     __shared__ int s_lvl[5];
     __shared__ int s_sb[NT + 1];                  // the tile's nodes' first segments
     __shared__ int s_lp[SEG_LDS], s_rp[SEG_LDS];  // local side prefixes of its first SEG_LDS segments
+    __shared__ Lvl s_L;                           // the last tile's level state
     const int t = threadIdx.x;
     if (t == 0) {
-        const bool ok = L->status == 0;   // a failed build has no active nodes
-        s_lvl[0] = ok ? L->scanA[par] : 0;
-        s_lvl[1] = L->scanAI[par];
-        s_lvl[2] = ok ? L->scanS[par] : 0;
+        const int st = L->status, sA = L->scanA[par], sAI = L->scanAI[par], sS = L->scanS[par], sR = L->scanR[par];
         s_lvl[3] = atomicAdd(&B.ctr[par], 1);
-        s_lvl[4] = L->scanR[par];
+        s_lvl[0] = st == 0 ? sA : 0;   // a failed build has no active nodes
+        s_lvl[1] = sAI;
+        s_lvl[2] = st == 0 ? sS : 0;
+        s_lvl[4] = sR;
     }
     __syncthreads();
     const int A = s_lvl[0], active_index = s_lvl[1], S = s_lvl[2];
     const bool repl_in = s_lvl[4], repl_out = A < JOIN_TEST_NODES;   // this level's keys, the next level's
-    const long long cap_nodes = L->cap_nodes;
     const bool es = empty_space && active_index != 0;   // the root level has no empty-space cuts
     const int ntiles = max(1, (A + NT - 1) / NT);
     // the next level's box keys: every possible child slot (created <= 2A),
     // before any scatter joins into them
-    {
-        key_reset(keys_next, 2ll * A, repl_out);
-    }
+    key_reset(keys_next, 2ll * A, repl_out);
     for (int tile = s_lvl[3]; tile < ntiles; tile = next_tile(&B.ctr[par], &s_tile, ntiles)) {
-        const int i0 = tile * NT, n = min(NT, A - i0);
+        const int i0 = tile * NT, n = min(NT, A - i0), i = i0 + t, node = active_index + i;
+        const bool last = tile == ntiles - 1, in_tile = t < n;
         // every node input first, then the node records (the stores would
         // otherwise hold back the next node's loads)
-        NodeIn in[NPT];
-#pragma unroll
-        for (int j = 0; j < NPT; ++j) {
-            const int li = NPT * t + j;
-            if (li < n) load_node(N, i0 + li, active_index + i0 + li, keys, repl_in, es, in[j]);
-        }
+        NodeIn in;
+        if (in_tile) load_node(N, i, node, keys, repl_in, es, in);
         for (int li = t; li <= n; li += LBS) s_sb[li] = n > 0 ? B.segbase[i0 + li] : 0;
-        int pl[NPT];
-#pragma unroll
-        for (int j = 0; j < NPT; ++j) {
-            const int li = NPT * t + j;
-            pl[j] = 0;
-            if (li < n) prepare_node(N, active_index + i0 + li, in[j], es, thr, pl[j]);
-        }
+        if (last)
+            for (int w = t; w < LvlMirror::NW; w += LBS)
+                reinterpret_cast<int *>(&s_L)[w] = reinterpret_cast<const int *>(L)[w];
+        int pl = 0, ax = AX_X, left_child = -1;
+        float sp = 0.0f;
+        f3 rMin = {0.0f, 0.0f, 0.0f}, rMax = rMin;
+        if (in_tile) prepare_node(N, node, in, es, thr, pl, ax, sp, rMin, rMax);
+        if (pl) left_child = N.children[in.parent].x;   // is the node its parent's left child
         __syncthreads();
         // the tile's segments [sb, se): the side counts' exclusive prefixes
         // inside the tile
         const int sb = s_sb[0], se = s_sb[n];
         int cL = 0, cR = 0;
-        for (int c0 = sb; c0 < se; c0 += NT) {
-            int v[2] = {0, 0}, sl[NPT], sr[NPT];
+        if (se - sb <= SEG_LDS) {
+            // up to 8 consecutive segments a thread, in one round
+            constexpr int PER = SEG_LDS / LBS;
+            const int per = (se - sb + LBS - 1) / LBS;
+            int sl[PER], sr[PER], v[2] = {0, 0};
 #pragma unroll
-            for (int j = 0; j < NPT; ++j) {
-                const int s = c0 + NPT * t + j;
-                sl[j] = s < se ? B.segL[s] : 0;
-                sr[j] = s < se ? B.segR[s] : 0;
-                v[0] += sl[j]; v[1] += sr[j];
+            for (int q = 0; q < PER; ++q) {
+                const int s = sb + t * per + q;
+                const bool has = q < per && s < se;
+                sl[q] = has ? B.segL[s] : 0;
+                sr[q] = has ? B.segR[s] : 0;
             }
+#pragma unroll
+            for (int q = 0; q < PER; ++q) { v[0] += sl[q]; v[1] += sr[q]; }
             int pre[2], tot[2];
             block_scan<2, LBS>(v, pre, tot, s_w);
-            int pl2 = cL + pre[0], pr2 = cR + pre[1];
 #pragma unroll
-            for (int j = 0; j < NPT; ++j) {
-                const int s = c0 + NPT * t + j;
-                if (s < se) {
-                    if (s - sb < SEG_LDS) { s_lp[s - sb] = pl2; s_rp[s - sb] = pr2; }
-                    else { B.segLoff[s] = pl2; B.segRoff[s] = pr2; }
-                }
-                pl2 += sl[j]; pr2 += sr[j];
+            for (int q = 0; q < PER; ++q) {
+                const int s = t * per + q;
+                if (q < per && sb + s < se) { s_lp[s] = pre[0]; s_rp[s] = pre[1]; }
+                pre[0] += sl[q]; pre[1] += sr[q];
             }
-            cL += tot[0]; cR += tot[1];
+            cL = tot[0]; cR = tot[1];
+        } else {
+            for (int c0 = sb; c0 < se; c0 += LBS) {
+                const int s = c0 + t;
+                int v[2] = {s < se ? B.segL[s] : 0, s < se ? B.segR[s] : 0};
+                int pre[2], tot[2];
+                block_scan<2, LBS>(v, pre, tot, s_w);
+                if (s < se) {
+                    if (s - sb < SEG_LDS) { s_lp[s - sb] = cL + pre[0]; s_rp[s - sb] = cR + pre[1]; }
+                    else { B.segLoff[s] = cL + pre[0]; B.segRoff[s] = cR + pre[1]; }
+                }
+                cL += tot[0]; cR += tot[1];
+            }
         }
         __syncthreads();   // the tile's local prefixes are visible to the whole block
         // a segment's local prefixes (se: the tile's totals)
@@ -997,29 +1017,23 @@ __global__ __launch_bounds__(LBS) void leaf_pass_kernel(NodePtrs N, Lvl *L, Leve
         // per node: empty-space nodes, children sizes and leaf flags
         // (CalcNodeChildSize, MarkNodeLeafs), leaf slots and refs, the
         // non-leaf children's segments
-        int v[7] = {0, 0, 0, 0, 0, 0, 0}, nl[NPT], nr[NPT], lb[NPT], rb[NPT];
-#pragma unroll
-        for (int j = 0; j < NPT; ++j) {
-            const int li = NPT * t + j;
-            nl[j] = nr[j] = 0;
-            lb[j] = rb[j] = 0;
-            if (li < n) {
-                const int b = s_sb[li], e = s_sb[li + 1];
-                lpre(b, lb[j], rb[j]);
-                if (e > b) {
-                    int le, re;
-                    lpre(e, le, re);
-                    nl[j] = le - lb[j];
-                    nr[j] = re - rb[j];
-                }
-                v[0] += 2 * __popc(pl[j]);
-                v[1] += nl[j] < LS;
-                v[2] += nr[j] < LS;
-                v[3] += nl[j] < LS ? nl[j] : 0;
-                v[4] += nr[j] < LS ? nr[j] : 0;
-                v[5] += nl[j] < LS ? 0 : (nl[j] + seg - 1) / seg;
-                v[6] += nr[j] < LS ? 0 : (nr[j] + seg - 1) / seg;
+        int v[7] = {0, 0, 0, 0, 0, 0, 0}, nl = 0, nr = 0, lb = 0, rb = 0;
+        if (in_tile) {
+            const int b = s_sb[t], e = s_sb[t + 1];
+            lpre(b, lb, rb);
+            if (e > b) {
+                int le, re;
+                lpre(e, le, re);
+                nl = le - lb;
+                nr = re - rb;
             }
+            v[0] = 2 * __popc(pl);
+            v[1] = nl < LS;
+            v[2] = nr < LS;
+            v[3] = nl < LS ? nl : 0;
+            v[4] = nr < LS ? nr : 0;
+            v[5] = nl < LS ? 0 : (nl + seg - 1) / seg;
+            v[6] = nr < LS ? 0 : (nr + seg - 1) / seg;
         }
         int pre[7], tot[7];
         block_scan<7, LBS>(v, pre, tot, s_w);
@@ -1032,19 +1046,16 @@ __global__ __launch_bounds__(LBS) void leaf_pass_kernel(NodePtrs N, Lvl *L, Leve
             if (t == 0) for (int k = 0; k < 8; ++k) s_ex[k] = ex[k];
         }
         __syncthreads();
+        int st = 0;
+        if (last && t == 0) st = __hip_atomic_load(&L->status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const int oL = (int)s_ex[0], oR = (int)s_ex[1], ereq = (int)s_ex[2];
         const int oSL = (int)(s_ex[7] & 0x7fffffff), oSR = (int)(s_ex[7] >> 31);
-        // the empty-space chains, only inside the capacity (a captured build
-        // that outgrew it fails in the plan below and writes nothing more)
-        const bool fits = (long long)active_index + A + ereq + tot[0] <= cap_nodes;
-        int r = pre[0];
-#pragma unroll
-        for (int j = 0; j < NPT; ++j) {
-            const int li = NPT * t + j;
-            if (li < n) {
-                if (pl[j] && fits) empty_chain_node_at(N, i0 + li, A, active_index, pl[j], ereq + r);
-                r += 2 * __popc(pl[j]);
-            }
+        if (in_tile) {
+            int4 *const rec = B.rec + 3ll * i;
+            rec[0] = make_int4(nl, nr, lb + oL, rb + oR);
+            rec[1] = make_int4((int)s_ex[3] + pre[1], (int)s_ex[4] + pre[2], (int)s_ex[5] + pre[3],
+                               (int)s_ex[6] + pre[4]);
+            rec[2] = make_int4(oSL + pre[5], oSR + pre[6], ax, __float_as_int(sp));
         }
         // the side offsets of the tile's segments, now global
         for (int s = sb + t; s < se; s += LBS) {
@@ -1053,23 +1064,12 @@ __global__ __launch_bounds__(LBS) void leaf_pass_kernel(NodePtrs N, Lvl *L, Leve
             B.segLoff[s] = l + oL;
             B.segRoff[s] = rr + oR;
         }
-        int p[6] = {(int)s_ex[3] + pre[1], (int)s_ex[4] + pre[2], (int)s_ex[5] + pre[3], (int)s_ex[6] + pre[4],
-                    oSL + pre[5], oSR + pre[6]};
-#pragma unroll
-        for (int j = 0; j < NPT; ++j) {
-            const int li = NPT * t + j;
-            if (li < n) {
-                B.lna[i0 + li] = make_int2(p[0], p[1]);
-                B.lref[i0 + li] = make_int2(p[2], p[3]);
-                B.lseg[i0 + li] = make_int2(p[4], p[5]);
-                B.nsz[i0 + li] = make_int4(nl[j], nr[j], lb[j] + oL, rb[j] + oR);
-                p[0] += nl[j] < LS; p[1] += nr[j] < LS;
-                p[2] += nl[j] < LS ? nl[j] : 0; p[3] += nr[j] < LS ? nr[j] : 0;
-                p[4] += nl[j] < LS ? 0 : (nl[j] + seg - 1) / seg;
-                p[5] += nr[j] < LS ? 0 : (nr[j] + seg - 1) / seg;
-            }
-        }
-        if (tile == ntiles - 1) {
+        // the empty-space chains, only inside the capacity (a captured build
+        // that outgrew it fails in the plan below and writes nothing more)
+        if (pl && (long long)active_index + A + ereq + tot[0] <= L->cap_nodes)
+            empty_chain_node_at(N, node, active_index + A + ereq + pre[0], pl, in.parent, left_child == node, rMin,
+                                rMax);
+        if (last) {
             if (t == 0) {
                 const int Lall = oL + cL, Rall = oR + cR, E = ereq + tot[0];
                 const int leafL = (int)s_ex[3] + tot[1], leafR = (int)s_ex[4] + tot[2];
@@ -1077,39 +1077,42 @@ __global__ __launch_bounds__(LBS) void leaf_pass_kernel(NodePtrs N, Lvl *L, Leve
                 const long long SL = (long long)oSL + tot[5], SR = (long long)oSR + tot[6];
                 B.segLoff[S] = Lall;
                 B.segRoff[S] = Rall;
+                if (st) lvl_fail(&s_L, st);
                 // the previous level's advance, this level's empty-space
                 // nodes and segments, then its children plan
-                plan_nodes(L, E, S);
-                if (!L->status) {
-                    const ChildPlan P = plan_children_totals(L, Lall, Rall, LL, LR, leafL + leafR);
+                plan_nodes(&s_L, E, S);
+                if (!s_L.status) {
+                    const ChildPlan P = plan_children_totals(&s_L, Lall, Rall, LL, LR, leafL + leafR);
                     if (P.status) {
-                        lvl_fail(L, P.status);
-                    } else if (SL + SR > L->cap_segs) {
-                        lvl_fail(L, PM_ERR_CAPACITY);
+                        lvl_fail(&s_L, P.status);
+                    } else if (SL + SR > s_L.cap_segs) {
+                        lvl_fail(&s_L, PM_ERR_CAPACITY);
                     } else {
-                        L->L_all = P.L_all; L->R_all = P.R_all; L->LL_all = P.LL_all; L->LR_all = P.LR_all;
-                        L->leaf_nodes = P.leaf_nodes; L->leafTri = P.leafTri; L->nextR = P.nextR;
-                        L->created = P.created; L->child_start = P.child_start; L->next_active = P.next_active;
-                        L->leaf_left = leafL;
-                        L->SL_all = (int)SL;
-                        L->advance = 1;
+                        s_L.L_all = P.L_all; s_L.R_all = P.R_all; s_L.LL_all = P.LL_all; s_L.LR_all = P.LR_all;
+                        s_L.leaf_nodes = P.leaf_nodes; s_L.leafTri = P.leafTri; s_L.nextR = P.nextR;
+                        s_L.created = P.created; s_L.child_start = P.child_start; s_L.next_active = P.next_active;
+                        s_L.leaf_left = leafL;
+                        s_L.SL_all = (int)SL;
+                        s_L.advance = 1;
                         // the next level as its passes will read it (advance_level's values)
-                        L->scanA[par ^ 1] = P.created;
-                        L->scanAI[par ^ 1] = L->nodes_size + 2 * L->A - P.created;
-                        L->scanS[par ^ 1] = (int)(SL + SR);
-                        L->scanR[par ^ 1] = repl_out;
+                        s_L.scanA[par ^ 1] = P.created;
+                        s_L.scanAI[par ^ 1] = s_L.nodes_size + 2 * s_L.A - P.created;
+                        s_L.scanS[par ^ 1] = (int)(SL + SR);
+                        s_L.scanR[par ^ 1] = repl_out;
                         B.segbase_n[P.created] = (int)(SL + SR);
                     }
                 }
                 B.ctr[par ^ 1] = 0;
             }
             __syncthreads();
+            for (int w = t; w < LvlMirror::NW; w += LBS)
+                reinterpret_cast<int *>(L)[w] = reinterpret_cast<const int *>(&s_L)[w];
+            // an eager build: the level state to the host
+            if (mirror) publish_level(&s_L, mirror, seq);
             // the next level's leaf pass starts with fresh status words
-            const int created = L->status ? 0 : L->created;
+            const int created = s_L.status ? 0 : s_L.created;
             const int nt = max(1, (created + NT - 1) / NT);
             for (int k = t; k < 8 * nt; k += LBS) B.lb_n[k] = 0ull;
-            // an eager build: the level state to the host
-            if (mirror) publish_level(L, mirror, seq);
         }
     }
 }
@@ -1129,21 +1132,20 @@ __device__ __forceinline__ void child_ids(const LevelPlan &P, int i, const int2 
     idR = P.child_start + (leafR ? lnaR : P.A + i - lnaR + P.leaf_nodes);
 }
 
-__device__ void write_children(const NodePtrs &N, const LevelPlan &P, const LevelBufs &B, int i, int propagate,
+__device__ void write_children(const NodePtrs &N, const LevelPlan &P, const LevelBufs &B, int i, const int4 &sz,
+                               const int4 &lf, const int4 &sg, const float4 &pmn, const float4 &pmx, int propagate,
                                int *__restrict__ leaf_ids) {
-    const int4 sz = B.nsz[i];
     const int sizes[2] = {sz.x, sz.y};
     const bool leaf[2] = {sizes[0] < P.LS, sizes[1] < P.LS};
-    const int2 ln = B.lna[i], lr = B.lref[i];
+    const int2 ln = make_int2(lf.x, lf.y), lr = make_int2(lf.z, lf.w);
     int ids[2];
     child_ids(P, i, ln, leaf[0], leaf[1], ids[0], ids[1]);
     const int split_addr[2] = {sz.z, P.L_all + sz.w};
     const int leaf_addr[2] = {lr.x, P.LL_all + lr.y};
     const int lna[2] = {ln.x, P.leaf_left + ln.y};
     const int par = P.active_index + i;
-    const int ax = N.info[par] & 3;
-    const float s = N.split[par];
-    const float4 pmn = N.bmin[par], pmx = N.bmax[par];
+    const int ax = sg.z;
+    const float s = __int_as_float(sg.w);
     for (int side = 0; side < 2; ++side) {
         const int id = ids[side];
         N.info[id] = LEAF; N.split[id] = 0.0f;
@@ -1166,7 +1168,7 @@ __device__ void write_children(const NodePtrs &N, const LevelPlan &P, const Leve
         }
         if (leaf[side]) leaf_ids[P.nleaf + lna[side]] = id;
         // a non-leaf child's first segment in the next level's table
-        else B.segbase_n[id - P.next_active] = side == 0 ? B.lseg[i].x : P.SL_all + B.lseg[i].y;
+        else B.segbase_n[id - P.next_active] = side == 0 ? sg.x : P.SL_all + sg.y;
     }
     N.children[par] = make_int2(ids[0], ids[1]);
 }
@@ -1177,48 +1179,56 @@ __device__ void write_children(const NodePtrs &N, const LevelPlan &P, const Leve
 // its non-leaf children's segments of the next level's table
 template <int SEGT, bool DIV>
 __device__ __forceinline__ void scatter_pass_segment(
-    const NodePtrs &N, const LevelPlan &P, const LevelBufs &B, int s, int propagate,
+    const NodePtrs &N, const LevelPlan &P, const LevelBufs &B, const int4 &r, int sL, int sR, int propagate,
     const float4 *__restrict__ rmin, const float4 *__restrict__ rmax,
     float4 *__restrict__ nmin, float4 *__restrict__ nmax, float4 *__restrict__ fmin,
     float4 *__restrict__ fmax, int *__restrict__ keys_next, int *__restrict__ leaf_ids, const DivideGeom &dg,
     bool join_test) {
     const int lane = threadIdx.x & 63;
-    const int i = B.seg_node[s];
-    const int start = B.seg_start[s], count = B.seg_count[s];
-    const int sL = B.segLoff[s], sR = B.segRoff[s];
+    const int i = __builtin_amdgcn_readfirstlane(r.x), start = __builtin_amdgcn_readfirstlane(r.y);
+    const int count = __builtin_amdgcn_readfirstlane(r.z);
+    const bool node_wave = __builtin_amdgcn_readfirstlane(r.w) == 0;   // the node's first segment
     const int node = P.active_index + i;
-    const int b = B.segbase[i];
-    const int4 nsz = B.nsz[i];
+    // the node's records, the first refs and (the node's wave) its box: one wait
+    const int4 nsz = B.rec[3ll * i], lf = B.rec[3ll * i + 1], sg = B.rec[3ll * i + 2];
+    constexpr int PRE = 2;
+    float4 pmn_r[PRE], pmx_r[PRE];
+#pragma unroll
+    for (int q = 0; q < PRE; ++q) {
+        const int j = q * 64 + lane;
+        const int k = start + (j < count ? j : 0);
+        pmn_r[q] = rmin[k];
+        pmx_r[q] = rmax[k];
+    }
+    float4 pmn = make_float4(0.0f, 0.0f, 0.0f, 0.0f), pmx = pmn;
+    if (node_wave || DIV) { pmn = N.bmin[node]; pmx = N.bmax[node]; }
     const int nl = nsz.x, nr = nsz.y;
     const bool leafL = nl < P.LS, leafR = nr < P.LS;
-    const int2 ln = B.lna[i], lr = B.lref[i];
+    const int2 ln = make_int2(lf.x, lf.y), lr = make_int2(lf.z, lf.w);
     int idL, idR;
     child_ids(P, i, ln, leafL, leafR, idL, idR);
-    if (s == b) {
+    if (node_wave) {
         // the node's wave: its two child records, and its non-leaf children's
         // segments (their refs start where the scatter below puts them)
-        if (lane == 0) write_children(N, P, B, i, propagate, leaf_ids);
-        const int2 ls = B.lseg[i];
+        if (lane == 0) write_children(N, P, B, i, nsz, lf, sg, pmn, pmx, propagate, leaf_ids);
         const bool leaf[2] = {leafL, leafR};
         const int sz[2] = {nl, nr}, ci[2] = {idL - P.next_active, idR - P.next_active};
         const int first[2] = {sL - lr.x, (P.L_all - P.LL_all) + sR - lr.y};
-        const int sbase[2] = {ls.x, P.SL_all + ls.y};
+        const int sbase[2] = {sg.x, P.SL_all + sg.y};
 #pragma unroll
         for (int side = 0; side < 2; ++side) {
             if (leaf[side]) continue;
             const int ns = (sz[side] + P.seg - 1) / P.seg;
             for (int k = lane; k < ns; k += 64)
-                write_segment(B.seg_node_n, B.seg_start_n, B.seg_count_n, sbase[side] + k, ci[side], first[side],
-                              sz[side], P.seg, k);
+                write_segment(B.seg_n, sbase[side] + k, ci[side], first[side], sz[side], P.seg, k);
         }
     }
     const int LLoff = lr.x + (leafL ? sL - nsz.z : 0);
     const int LRoff = lr.y + (leafR ? sR - nsz.w : 0);
     // one chunk per wave: its node's axis and plane are wave-uniform
-    const int ax = __builtin_amdgcn_readfirstlane(N.info[node]);
-    const float sp = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(N.split[node])));
-    f3 nmn = {0.0f, 0.0f, 0.0f}, nmx = nmn;
-    if (DIV) { nmn = mk3(N.bmin[node]); nmx = mk3(N.bmax[node]); }
+    const int ax = __builtin_amdgcn_readfirstlane(sg.z);
+    const float sp = __int_as_float(__builtin_amdgcn_readfirstlane(sg.w));
+    const f3 nmn = mk3(pmn), nmx = mk3(pmx);   // (DIV only)
     float4 *dLmin, *dLmax, *dRmin, *dRmax;
     long long bL, bR;
     if (leafL) { dLmin = fmin; dLmax = fmax; bL = (long long)P.ulp + LLoff; }
@@ -1230,19 +1240,11 @@ __device__ __forceinline__ void scatter_pass_segment(
     int l0 = fkey(F_INF), l1 = l0, l2 = l0, l3 = fkey(-F_INF), l4 = l3, l5 = l3;
     int r0 = l0, r1 = l0, r2 = l0, r3 = l3, r4 = l3, r5 = l3;
     // groups of iterations: a group's refs are loaded first (lanes past the
-    // chunk re-read its first ref), then classified and written; groups of 4
-    // while the chunk has that many iterations left, then groups of 2 (more
-    // would cost the kernel its fifth wave per SIMD)
-    auto group = [&](int g0, auto GC) {
+    // chunk re-read its first ref), then classified and written; the two
+    // loaded above, then groups of 4 while the chunk has that many iterations
+    // left, then groups of 2 (more would cost the kernel its fifth wave per SIMD)
+    auto write_group = [&](int g0, auto &gmn, auto &gmx, auto GC) {
         constexpr int G = decltype(GC)::value;
-        float4 gmn[G], gmx[G];
-#pragma unroll
-        for (int q = 0; q < G; ++q) {
-            const int jq = (g0 + q) * 64 + lane;
-            const int k = start + (jq < count ? jq : 0);
-            gmn[q] = rmin[k];
-            gmx[q] = rmax[k];
-        }
 #pragma unroll
         for (int q = 0; q < G; ++q) {
             const int j = (g0 + q) * 64 + lane;
@@ -1283,9 +1285,22 @@ __device__ __forceinline__ void scatter_pass_segment(
             rr += __popcll(brm);
         }
     };
+    auto group = [&](int g0, auto GC) {
+        constexpr int G = decltype(GC)::value;
+        float4 gmn[G], gmx[G];
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            const int jq = (g0 + q) * 64 + lane;
+            const int k = start + (jq < count ? jq : 0);
+            gmn[q] = rmin[k];
+            gmx[q] = rmax[k];
+        }
+        write_group(g0, gmn, gmx, GC);
+    };
     constexpr int GB = SEGT / 64 < 4 ? SEGT / 64 : 4;
     const int its = (count + 63) >> 6;   // wave-uniform
-    int g0 = 0;
+    write_group(0, pmn_r, pmx_r, std::integral_constant<int, PRE>{});
+    int g0 = PRE;
     for (; g0 + GB <= its; g0 += GB) group(g0, std::integral_constant<int, GB>{});
     for (; g0 < its; g0 += 2) group(g0, std::integral_constant<int, 2>{});
     const bool doL = !leafL && rl > 0, doR = !leafR && rr > 0;   // wave-uniform
@@ -1323,6 +1338,10 @@ __device__ __forceinline__ void scatter_pass(const NodePtrs N, const Lvl *L, con
                                              float4 *__restrict__ nmin, float4 *__restrict__ nmax,
                                              float4 *__restrict__ fmin, float4 *__restrict__ fmax,
                                              int *__restrict__ keys_next, int *__restrict__ leaf_ids, DivideGeom dg) {
+    // (the wave's first segment, loaded with the level's plan)
+    const int s0 = __builtin_amdgcn_readfirstlane(wave_index()), sc0 = min(s0, B.seg_last);
+    int4 r = B.seg[sc0];
+    int sL = B.segLoff[sc0], sR = B.segRoff[sc0];
     if (L->status) return;
     LevelPlan P;
     P.A = L->A; P.active_index = L->active_index; P.child_start = L->child_start; P.next_active = L->next_active;
@@ -1330,12 +1349,16 @@ __device__ __forceinline__ void scatter_pass(const NodePtrs N, const Lvl *L, con
     P.ulp = L->final_refs; P.nleaf = L->nleaf; P.LS = LS;
     P.SL_all = L->SL_all; P.seg = seg;
     const int S = L->S;
-    for (int s = wave_index(); s < S; s += wave_count())
-        scatter_pass_segment<SEGT, DIV>(N, P, B, s, propagate, rmin, rmax, nmin, nmax, fmin, fmax, keys_next,
+    for (int s = s0; s < S; s += wave_count()) {
+        if (s != s0) { r = B.seg[s]; sL = B.segLoff[s]; sR = B.segRoff[s]; }
+        scatter_pass_segment<SEGT, DIV>(N, P, B, r, sL, sR, propagate, rmin, rmax, nmin, nmax, fmin, fmax, keys_next,
                                         leaf_ids, dg, P.A < JOIN_TEST_NODES);
+    }
     // nodes without refs (an empty mesh's root) have no segment to write their children
     GRID_STRIDE(i, P.A)
-        if (B.segbase[i + 1] == B.segbase[i]) write_children(N, P, B, i, propagate, leaf_ids);
+        if (B.segbase[i + 1] == B.segbase[i])
+            write_children(N, P, B, i, B.rec[3ll * i], B.rec[3ll * i + 1], B.rec[3ll * i + 2],
+                           N.bmin[P.active_index + i], N.bmax[P.active_index + i], propagate, leaf_ids);
 }
 
 template <int SEGT>
@@ -2268,8 +2291,7 @@ namespace {
 // scan: its S segments follow from ntris and are written here too.
 __global__ void build_init_kernel(Lvl *L, Lvl v, NodePtrs N, const int *__restrict__ off, int M, int ntris, int *keys,
                                   int repl, unsigned long long *lb0, unsigned long long *lb1, int nlb, int *ctr,
-                                  int *__restrict__ segbase, int *__restrict__ sn, int *__restrict__ ss,
-                                  int *__restrict__ sc, int S, int seg) {
+                                  int *__restrict__ segbase, int4 *__restrict__ table, int S, int seg) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *L = v;
     GRID_STRIDE(m, M) {
         zero_node(N, m);
@@ -2282,7 +2304,7 @@ __global__ void build_init_kernel(Lvl *L, Lvl v, NodePtrs N, const int *__restri
             segbase[0] = 0;
             segbase[1] = S;
         }
-        GRID_STRIDE(k, S) write_segment(sn, ss, sc, k, 0, 0, ntris, seg, k);
+        GRID_STRIDE(k, S) write_segment(table, k, 0, 0, ntris, seg, k);
     }
     key_reset(keys, M, repl);
     GRID_STRIDE(k, nlb) {
@@ -2385,12 +2407,10 @@ void reserve_first(pm_ctx *ctx, int N, int M, int seg, hipStream_t s) {
         sc.ref_max[q].reserve((size_t)r + 1, s);
         sc.keys[q].reserve((size_t)std::max(12 * a, key_words_host(2 * JOIN_TEST_NODES, true)) + 6, s);
         sc.node_segbase[q].reserve((size_t)(2 * a) + 2, s);
-        for (DevBuf<int> *b : {&sc.seg_node[q], &sc.seg_start[q], &sc.seg_count[q]})
-            b->reserve((size_t)(2 * a + r / seg) + 1, s);
+        sc.segs[q].reserve((size_t)(2 * a + r / seg) + 1, s);
     }
     for (DevBuf<int> *b : {&sc.segL, &sc.segR, &sc.segLoff, &sc.segRoff}) b->reserve((size_t)(a + r / seg) + 1, s);
-    sc.node_lna.reserve((size_t)a + 1, s); sc.node_lref.reserve((size_t)a + 1, s);
-    sc.node_lseg.reserve((size_t)a + 1, s); sc.node_sz.reserve((size_t)a + 1, s);
+    sc.node_rec.reserve(3 * (size_t)a + 3, s);
     sc.prim_min.reserve((size_t)r + 1, s); sc.prim_max.reserve((size_t)r + 1, s);
     ctx->leaf_ids.reserve((size_t)n / 2 + 2 * M, s);
     ctx->nodes.reserve((size_t)(n + n / 2) + 1024 + 16 * M, s, 0);
@@ -2450,7 +2470,7 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
     const long long S_now = graph ? caps->segs : M + (N + seg - 1) / seg;
     if (!graph) {
         sc.node_segbase[0].reserve((size_t)M + 1, s);
-        for (DevBuf<int> *b : {&sc.seg_node[0], &sc.seg_start[0], &sc.seg_count[0]}) b->reserve(S_now + 1, s);
+        sc.segs[0].reserve(S_now + 1, s);
     }
     const int S1 = M == 1 ? (N + seg - 1) / seg : 0;   // a single root's segments
     h.scanS[0] = S1;
@@ -2461,8 +2481,7 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
                                       (long long)grid_for(nlb, BS, 64)});
         build_init_kernel<<<(int)g, BS, 0, s>>>(L, h, node_ptrs(ctx), off_dev, M, N, sc.keys[0].ptr, repl0,
                                                  sc.lb_words[0].ptr, sc.lb_words[1].ptr, nlb, sc.lb_ctr.ptr,
-                                                 sc.node_segbase[0].ptr, sc.seg_node[0].ptr, sc.seg_start[0].ptr,
-                                                 sc.seg_count[0].ptr, h.status ? 0 : S1, seg);
+                                                 sc.node_segbase[0].ptr, sc.segs[0].ptr, h.status ? 0 : S1, seg);
         PM_LAUNCH_CHECK();
     }
     if (N > 0) {
@@ -2474,16 +2493,17 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
 
     const DivideGeom dg = {prm.split_method == PM_SPLIT_DIVIDE ? P0 : nullptr, P1, P2};
     const bool div = dg.p0 != nullptr;
-    auto level_bufs = [&](int par) {
+    auto level_bufs = [&](int par, long long S_bound) {
         const int q = par ^ 1;
         LevelBufs B;
         B.segbase = sc.node_segbase[par].ptr;
-        B.seg_node = sc.seg_node[par].ptr; B.seg_start = sc.seg_start[par].ptr; B.seg_count = sc.seg_count[par].ptr;
+        B.seg = sc.segs[par].ptr;
+        B.seg_last = (int)S_bound;
         B.segL = sc.segL.ptr; B.segR = sc.segR.ptr;
         B.segLoff = sc.segLoff.ptr; B.segRoff = sc.segRoff.ptr;
-        B.lna = sc.node_lna.ptr; B.lref = sc.node_lref.ptr; B.lseg = sc.node_lseg.ptr; B.nsz = sc.node_sz.ptr;
+        B.rec = sc.node_rec.ptr;
         B.segbase_n = sc.node_segbase[q].ptr;
-        B.seg_node_n = sc.seg_node[q].ptr; B.seg_start_n = sc.seg_start[q].ptr; B.seg_count_n = sc.seg_count[q].ptr;
+        B.seg_n = sc.segs[q].ptr;
         B.lb = sc.lb_words[par].ptr; B.lb_n = sc.lb_words[q].ptr;
         B.ctr = sc.lb_ctr.ptr;
         return B;
@@ -2491,8 +2511,7 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
 
     if (M > 1) {
         root_segments_kernel<<<(int)tiles(M, NT), LBS, 0, s>>>(node_ptrs(ctx), L, sc.node_segbase[0].ptr,
-                                                               sc.seg_node[0].ptr, sc.seg_start[0].ptr,
-                                                               sc.seg_count[0].ptr, sc.lb_words[1].ptr,
+                                                               sc.segs[0].ptr, sc.lb_words[1].ptr,
                                                                sc.lb_ctr.ptr + 1, M, seg);
         PM_LAUNCH_CHECK();
     }
@@ -2521,8 +2540,7 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
         const long long A_g = graph ? caps->active : A_now, S_g = graph ? caps->segs : b.S;
         if (!graph) {
             for (DevBuf<int> *q : {&sc.segL, &sc.segR, &sc.segLoff, &sc.segRoff}) q->reserve(b.S + 1, s);
-            sc.node_lna.reserve(A_now + 1, s); sc.node_lref.reserve(A_now + 1, s); sc.node_lseg.reserve(A_now + 1, s);
-            sc.node_sz.reserve(A_now + 1, s);
+            sc.node_rec.reserve(3 * (size_t)A_now + 3, s);
             const LevelSizes w = b.next_bound(seg);   // what the level may write
             nodes.reserve((size_t)w.nodes + 1, s, (size_t)b.nodes);
             // (replicated if the level turns out to have few nodes)
@@ -2534,9 +2552,9 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
             sc.prim_max.reserve((size_t)w.fin + 1, s, (size_t)b.fin);
             ctx->leaf_ids.reserve((size_t)w.nleaf + 1, s, (size_t)b.nleaf);
             sc.ref_min[nxt].reserve((size_t)w.R + 1, s); sc.ref_max[nxt].reserve((size_t)w.R + 1, s);
-            for (DevBuf<int> *q : {&sc.seg_node[nxt], &sc.seg_start[nxt], &sc.seg_count[nxt]}) q->reserve(w.S + 1, s);
+            sc.segs[nxt].reserve(w.S + 1, s);
         }
-        const LevelBufs B = level_bufs(par);
+        const LevelBufs B = level_bufs(par, S_g);
         const NodePtrs NP = node_ptrs(ctx);
         launch_classify_pass(seg, div, grid_for(S_g, WPB, graph ? 2048 : INT_MAX), s, (const Lvl *)L, B, par,
                              (const int *)sc.keys[par].ptr, (const float4 *)sc.ref_min[par].ptr,
@@ -2758,12 +2776,9 @@ void reserve_build_caps(pm_ctx *ctx, const BuildSizes &caps, int N, hipStream_t 
     }
     for (int q = 0; q < 2; ++q) {
         sc.node_segbase[q].reserve((size_t)caps.active + 1, s);
-        for (DevBuf<int> *b : {&sc.seg_node[q], &sc.seg_start[q], &sc.seg_count[q]}) b->reserve((size_t)caps.segs + 1, s);
+        sc.segs[q].reserve((size_t)caps.segs + 1, s);
     }
-    sc.node_lna.reserve((size_t)caps.active + 1, s);
-    sc.node_lref.reserve((size_t)caps.active + 1, s);
-    sc.node_lseg.reserve((size_t)caps.active + 1, s);
-    sc.node_sz.reserve((size_t)caps.active + 1, s);
+    sc.node_rec.reserve(3 * (size_t)caps.active + 3, s);
     for (DevBuf<int> *b : {&sc.segL, &sc.segR, &sc.segLoff, &sc.segRoff}) b->reserve((size_t)caps.segs + 1, s);
     // the leaf passes' status words (8 per tile of NT nodes; the roots' scan
     // uses parity 1's, M <= caps.active)
@@ -2871,8 +2886,7 @@ std::vector<void **> graph_buffers(pm_ctx *ctx) {
         (void **)&a.parent.ptr, (void **)&ctx->prim_indices.ptr, (void **)&ctx->leaf_ids.ptr,
         (void **)&ctx->packed.ptr, (void **)&ctx->leaf_rec.ptr, (void **)&ctx->leaf_tris.ptr, (void **)&sc.prim_min.ptr,
         (void **)&sc.prim_max.ptr, (void **)&sc.segL.ptr, (void **)&sc.segR.ptr,
-        (void **)&sc.segLoff.ptr, (void **)&sc.segRoff.ptr, (void **)&sc.node_lna.ptr, (void **)&sc.node_lref.ptr,
-        (void **)&sc.node_lseg.ptr, (void **)&sc.node_sz.ptr, (void **)&sc.lb_ctr.ptr, (void **)&sc.prims_part.ptr, (void **)&sc.areas.ptr, (void **)&sc.lower_flag.ptr,
+        (void **)&sc.segLoff.ptr, (void **)&sc.segRoff.ptr, (void **)&sc.node_rec.ptr, (void **)&sc.lb_ctr.ptr, (void **)&sc.prims_part.ptr, (void **)&sc.areas.ptr, (void **)&sc.lower_flag.ptr,
         (void **)&sc.lower_off.ptr, (void **)&sc.lower_sets.ptr, (void **)&sc.lower_careas.ptr,
         (void **)&sc.lower_list.ptr, (void **)&sc.tri_rec.ptr, (void **)&ctx->graph_off.ptr, (void **)&sc.lvl.ptr};
     for (int i = 0; i < 2; ++i) {
@@ -2880,9 +2894,7 @@ std::vector<void **> graph_buffers(pm_ctx *ctx) {
         v.push_back((void **)&sc.ref_max[i].ptr);
         v.push_back((void **)&sc.keys[i].ptr);
         v.push_back((void **)&sc.node_segbase[i].ptr);
-        v.push_back((void **)&sc.seg_node[i].ptr);
-        v.push_back((void **)&sc.seg_start[i].ptr);
-        v.push_back((void **)&sc.seg_count[i].ptr);
+        v.push_back((void **)&sc.segs[i].ptr);
         v.push_back((void **)&sc.lb_words[i].ptr);
     }
     for (int i = 0; i < 3; ++i) v.push_back((void **)&sc.scan_tmp[i].ptr);

@@ -199,12 +199,10 @@ struct BuildScratch {
     DevBuf<float4> prim_min, prim_max;         // final (upper leaf) refs
     DevBuf<int> keys[2];                        // 6 ordered-int box keys per active node
     DevBuf<int> node_segbase[2];                // per active node: first segment (by level parity)
-    DevBuf<int> seg_node[2], seg_start[2], seg_count[2];   // segment tables (by level parity)
+    DevBuf<int4> segs[2];                       // segment tables (by level parity)
     DevBuf<int> segL, segR;                     // per segment: left / right refs
     DevBuf<int> segLoff, segRoff;               // per segment: left / right refs before it
-    DevBuf<int2> node_lna, node_lref;           // per active node: leaf slots and leaf refs before it (left, right)
-    DevBuf<int2> node_lseg;                     // per active node: its non-leaf children's segments before it
-    DevBuf<int4> node_sz;                       // per active node: children sizes, side offsets of its first segment
+    DevBuf<int4> node_rec;                      // per active node: 3 records for the scatter pass (LevelBufs::rec)
     DevBuf<unsigned long long> lb_words[2];     // look-back status words of the leaf passes (by level parity)
     DevBuf<int> lb_ctr;                         // their tile tickets (by level parity)
     DevBuf<int> scan_tmp[3];                    // block sums for scans, per level
