@@ -69,6 +69,7 @@ struct ScanIO {
     int n_mult[K];
 };
 
+template <bool TRACK>
 __device__ void plan_nodes(Lvl *L, int E, int S);
 __host__ __device__ void lvl_fail(Lvl *L, int code);
 __host__ __device__ void advance_level(Lvl *L);
@@ -634,7 +635,7 @@ struct LevelBufs {
     int *segbase_n;            // the same for the next level
     int4 *seg_n;
     unsigned long long *lb, *lb_n;   // look-back words of this level's leaf pass and the next's
-    int *ctr;                  // leaf pass tickets by level parity
+    int *ctr;                  // leaf pass tickets by level parity, then the largest children by level parity
 };
 
 // what prepare_node reads of active node i: its six box keys and (empty-space
@@ -675,22 +676,26 @@ __device__ __forceinline__ void node_split(f3 rMin, f3 rMax, int &ax, float &sp)
     ax = zHigher ? AX_Z : (yAboveX ? AX_Y : AX_X);
 }
 
+// CalcEmptySpaceSplits (EmptySpaceSplitting.h:10-70): the sides on which the
+// reduced box leaves more than thr of the given box empty
+__device__ __forceinline__ int empty_planes(f3 rMin, f3 rMax, f3 pMin, f3 pMax, float thr) {
+    int pl = 0;
+    if (rMin.x - pMin.x > thr * (pMax.x - pMin.x)) pl |= 1;
+    if (rMin.y - pMin.y > thr * (pMax.y - pMin.y)) pl |= 2;
+    if (rMin.z - pMin.z > thr * (pMax.z - pMin.z)) pl |= 4;
+    if (pMax.x - rMax.x > thr * (pMax.x - pMin.x)) pl |= 8;
+    if (pMax.y - rMax.y > thr * (pMax.y - pMin.y)) pl |= 16;
+    if (pMax.z - rMax.z > thr * (pMax.z - pMin.z)) pl |= 32;
+    return pl;
+}
+
 // ReduceAabb result -> node box, CalcEmptySpaceSplits (EmptySpaceSplitting.h:
 // 10-70) and the split plane for an active node, from what load_node read
 __device__ __forceinline__ void prepare_node(const NodePtrs &N, int node, const NodeIn &v, bool empty_space,
                                              float thr, int &pl, int &ax, float &sp, f3 &rMin, f3 &rMax) {
     rMin = {unkey(v.k01.x), unkey(v.k01.y), unkey(v.k23.x)};
     rMax = {unkey(v.k23.y), unkey(v.k45.x), unkey(v.k45.y)};
-    pl = 0;
-    if (empty_space) {
-        const f3 pMin = mk3(v.pmn), pMax = mk3(v.pmx);
-        if (rMin.x - pMin.x > thr * (pMax.x - pMin.x)) pl |= 1;
-        if (rMin.y - pMin.y > thr * (pMax.y - pMin.y)) pl |= 2;
-        if (rMin.z - pMin.z > thr * (pMax.z - pMin.z)) pl |= 4;
-        if (pMax.x - rMax.x > thr * (pMax.x - pMin.x)) pl |= 8;
-        if (pMax.y - rMax.y > thr * (pMax.y - pMin.y)) pl |= 16;
-        if (pMax.z - rMax.z > thr * (pMax.z - pMin.z)) pl |= 32;
-    }
+    pl = empty_space ? empty_planes(rMin, rMax, mk3(v.pmn), mk3(v.pmx), thr) : 0;
     N.bmin[node] = make_float4(rMin.x, rMin.y, rMin.z, 0.0f);
     N.bmax[node] = make_float4(rMax.x, rMax.y, rMax.z, 0.0f);
     node_split(rMin, rMax, ax, sp);
@@ -921,6 +926,9 @@ constexpr int SEG_LDS = 2048;
 // nodes (nothing else writes the state in this pass but a failed look-back its
 // status, which is looked at again), and stores and publishes it from there; a
 // node's parent and its side are loaded before the look-back, not after it.
+// TRACK: the largest node of the next level too, for the host's choice of
+// subtrees (without it the pass is shorter).
+template <bool TRACK>
 __global__ __launch_bounds__(LBS) void leaf_pass_kernel(NodePtrs N, Lvl *L, LevelBufs B, int par, int LS, int seg,
                                                        const int *__restrict__ keys, int *__restrict__ keys_next,
                                                        int empty_space, float thr, LvlMirror::Rec *mirror,
@@ -933,8 +941,10 @@ __global__ __launch_bounds__(LBS) void leaf_pass_kernel(NodePtrs N, Lvl *L, Leve
     __shared__ int s_sb[NT + 1];                  // the tile's nodes' first segments
     __shared__ int s_lp[SEG_LDS], s_rp[SEG_LDS];  // local side prefixes of its first SEG_LDS segments
     __shared__ Lvl s_L;                           // the last tile's level state
+    __shared__ int s_max;                         // largest non-leaf child of the block's tiles (TRACK)
     const int t = threadIdx.x;
     if (t == 0) {
+        if (TRACK) s_max = 0;
         const int st = L->status, sA = L->scanA[par], sAI = L->scanAI[par], sS = L->scanS[par], sR = L->scanR[par];
         s_lvl[3] = atomicAdd(&B.ctr[par], 1);
         s_lvl[0] = st == 0 ? sA : 0;   // a failed build has no active nodes
@@ -1035,8 +1045,17 @@ __global__ __launch_bounds__(LBS) void leaf_pass_kernel(NodePtrs N, Lvl *L, Leve
             v[5] = nl < LS ? 0 : (nl + seg - 1) / seg;
             v[6] = nr < LS ? 0 : (nr + seg - 1) / seg;
         }
+        if (TRACK) {   // the largest node of the next level
+            const int big = wave_max(max(nl < LS ? 0 : nl, nr < LS ? 0 : nr));
+            if ((t & 63) == 0) atomicMax(&s_max, big);
+        }
         int pre[7], tot[7];
         block_scan<7, LBS>(v, pre, tot, s_w);
+        if (TRACK && ntiles > 1 && t == 0) {
+            // joined (and the join waited for) before the tile's counts are published
+            const int old = atomicMax(&B.ctr[2 + par], s_max);
+            asm volatile("" ::"v"(old) : "memory");
+        }
         if (t < 64) {
             // the two segment counts share a word (each total < 2^31)
             const long long agg[8] = {cL, cR, tot[0], tot[1], tot[2], tot[3], tot[4],
@@ -1077,10 +1096,14 @@ __global__ __launch_bounds__(LBS) void leaf_pass_kernel(NodePtrs N, Lvl *L, Leve
                 const long long SL = (long long)oSL + tot[5], SR = (long long)oSR + tot[6];
                 B.segLoff[S] = Lall;
                 B.segRoff[S] = Rall;
+                if (TRACK)
+                    s_L.max_child = ntiles > 1 ? __hip_atomic_load(&B.ctr[2 + par], __ATOMIC_RELAXED,
+                                                                   __HIP_MEMORY_SCOPE_AGENT)
+                                               : s_max;
                 if (st) lvl_fail(&s_L, st);
                 // the previous level's advance, this level's empty-space
                 // nodes and segments, then its children plan
-                plan_nodes(&s_L, E, S);
+                plan_nodes<TRACK>(&s_L, E, S);
                 if (!s_L.status) {
                     const ChildPlan P = plan_children_totals(&s_L, Lall, Rall, LL, LR, leafL + leafR);
                     if (P.status) {
@@ -1103,6 +1126,7 @@ __global__ __launch_bounds__(LBS) void leaf_pass_kernel(NodePtrs N, Lvl *L, Leve
                     }
                 }
                 B.ctr[par ^ 1] = 0;
+                if (TRACK) B.ctr[2 + (par ^ 1)] = 0;
             }
             __syncthreads();
             for (int w = t; w < LvlMirror::NW; w += LBS)
@@ -1391,7 +1415,10 @@ __host__ __device__ void lvl_fail(Lvl *L, int code) {
 }
 
 // in the leaf pass's last tile: the previous level's advance, then the
-// empty-space nodes and segments of the level
+// empty-space nodes and segments of the level (an instance for each of the
+// pass's: shared, or forced inline, it leaves the pass 3% more instructions,
+// 0.7 us a level)
+template <bool TRACK>
 __device__ void plan_nodes(Lvl *L, int E, int S) {
     advance_level(L);
     // a failed advance (depth) has zeroed the level: E and S, counted over
@@ -1425,6 +1452,477 @@ __host__ __device__ void advance_level(Lvl *L) {
     L->R = L->nextR;
     L->level += 1;
     if (L->A > 0 && L->level >= L->max_levels) lvl_fail(L, PM_ERR_DEPTH);
+}
+
+// ================================================================== subtrees
+// On a small level (SUB_REFS) a pass takes the time of its chain of dependent
+// loads, some 9 us with its launch, whatever it does.  So once no active node
+// holds more than SUB_MAX refs, the rest of a small build's upper stage takes
+// three steps instead of three launches a level: subtree_kernel builds every
+// active node's subtree, a block each, out of order and without the final
+// numbering; number_pass_kernel, one launch a level, gives the nodes their
+// numbers in level order and writes them; leaf_move_kernel puts the leaves'
+// refs where the numbering says.  A ref's box at a node is its box at the
+// subtree's root clipped by the planes above the node, so a subtree keeps its
+// root's boxes in LDS and passes 16-bit indices down; a ref goes back to memory
+// once, when it reaches a leaf.
+// The nodes of a level are numbered by scans over the nodes before them, which
+// need the level's totals; the blocks add those up as they build, so the number
+// passes run back to back with nothing but look-backs between tiles.
+// What the subtrees cannot hold (a list, node or level bound passed) sets
+// `fail`, and the levels above go on as if the subtrees had not been tried:
+// they write only buffers of their own and the next level's refs.
+// A wave's node is a chain of LDS round trips and wave reductions (about 1.5
+// us) and a block's depth as long as its busiest wave, so the blocks have as
+// many waves as a depth has nodes: 16 and 8 (8 and 4 measured 2% slower on
+// builds of 5,000 to 100,000 triangles).  Where a level fills the device it is
+// instruction issue that counts, about 800 instructions a node against the
+// level passes' streaming: 1,000,002 triangles 1.41 ms without subtrees and
+// 1.54 ms with them, hence SUB_REFS.
+// Rebuilds, before and after: a 5,316-triangle room 702 -> 570 us, soups of
+// 2,000 / 10,000 / 100,000 triangles 328 / 446 / 650 -> 260 / 350 / 603 us, a
+// 31,752-triangle terrain 430 -> 350 us.
+constexpr int SUB_SMALL = 512;         // refs up to which a subtree goes to a block with less LDS (28 KB)
+constexpr int SUB_MAX = 1280;          // most refs a node may hold (64 KB)
+constexpr int SUB_GROW = 4;            // leaf ref slots per ref of a subtree's root
+constexpr int SUB_ARENA = 2;           // leaf ref slots per ref for the subtrees that outgrow theirs
+constexpr int SUB_COPIES = 64;         // copies of the levels' totals the blocks add into
+static_assert(SUB_LEVELS * SUB_COUNTS + 1 == SUB_WORDS, "the totals and the failure flag");
+
+// a node to build: list entries [base, base + n) of its depth's parity; the box
+// its parent gives it (floats) and the planes above it (keys)
+struct SubItem {
+    int base, n, slot;
+    f3 mn, mx;
+    int c0, c1, c2, c3, c4, c5;
+};
+
+// CAP refs at the root, LIST list entries and NODES nodes at one depth
+template <int CAP, int LIST, int NODES>
+struct SubShared {
+    static constexpr int nodes = NODES, entries = LIST;
+    int key[6][CAP];                   // the root's refs: box keys
+    unsigned short list[2][LIST];      // by depth parity
+    int4 item[2][NODES][4];            // a SubItem's words
+    int tot[SUB_LEVELS * SUB_COUNTS];
+    int cnt[2], used[2], slots, leaf, fail;   // nodes and list entries by depth parity
+};
+
+struct SubArgs {
+    const float4 *smin, *smax;         // the level's refs
+    float4 *xmin, *xmax;               // leaf refs
+    long long xcap;                    // refs they hold
+    int4 *rec;                         // per slot: box min | left size, box max | right size,
+                                       // left and right child (slot, or the leaf's first ref), axis, plane bits
+    int *slot;                         // per active node of the level: its slot
+    int *tot, *ctl;                    // totals (SUB_COPIES copies); ctl: failure flag, arena refs handed out
+    int active_index, R, LS, seg;
+    int empty_space;
+    float thr;
+};
+
+// (one lane writes; every lane reads the same words)
+template <class SH>
+__device__ __forceinline__ void sub_put(SH &sh, int d, int k, SubItem it) {
+    int4 *const w = sh.item[d & 1][k];
+    w[0] = make_int4(it.base, it.n, it.slot, 0);
+    w[1] = make_int4(__float_as_int(it.mn.x), __float_as_int(it.mn.y), __float_as_int(it.mn.z),
+                     __float_as_int(it.mx.x));
+    w[2] = make_int4(__float_as_int(it.mx.y), __float_as_int(it.mx.z), it.c0, it.c1);
+    w[3] = make_int4(it.c2, it.c3, it.c4, it.c5);
+}
+
+template <class SH>
+__device__ __forceinline__ SubItem sub_get(const SH &sh, int d, int k) {
+    const int4 *const w = sh.item[d & 1][k];
+    const int4 a = w[0], b = w[1], c = w[2], e = w[3];
+    auto word = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    auto real = [](int v) { return __int_as_float(__builtin_amdgcn_readfirstlane(v)); };
+    return SubItem{word(a.x), word(a.y), word(a.z), {real(b.x), real(b.y), real(b.z)},
+                   {real(b.w), real(c.x), real(c.y)}, word(c.z), word(c.w), word(e.x), word(e.y), word(e.z),
+                   word(e.w)};
+}
+
+__device__ __forceinline__ int pick3(int ax, int x, int y, int z) { return ax == AX_X ? x : ax == AX_Y ? y : z; }
+
+// One wave builds one node: its box, plane and sides, its children's refs
+// (CalcEmptySpaceSplits, CalcUpperNodeSplitInfo, SetSplitSide and
+// SplitTriangles as in the level passes).  HOLD: up to 64 G refs, read once and
+// held in registers; otherwise any number, read three times.  Its non-leaf
+// children are nodes of the next depth.
+template <bool HOLD, int G, class SH>
+__device__ __forceinline__ void sub_node(const SubArgs &a, SH &sh, const SubItem &it, int d, int start, int count,
+                                         int slot0, int slot_cap) {
+    const int lane = __lane_id();
+    const int n = it.n;
+    const unsigned short *const list = sh.list[d & 1] + it.base;
+    unsigned short *const out = sh.list[(d & 1) ^ 1];
+    int ix[G], k0[G], k1[G], k2[G], k3[G], k4[G], k5[G];
+    auto load = [&](int it0) {
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            const int j = (it0 + q) * 64 + lane;
+            ix[q] = list[j < n ? j : 0];
+        }
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            k0[q] = max(sh.key[0][ix[q]], it.c0); k1[q] = max(sh.key[1][ix[q]], it.c1);
+            k2[q] = max(sh.key[2][ix[q]], it.c2); k3[q] = min(sh.key[3][ix[q]], it.c3);
+            k4[q] = min(sh.key[4][ix[q]], it.c4); k5[q] = min(sh.key[5][ix[q]], it.c5);
+        }
+    };
+    const int its = (n + 63) >> 6;
+    // (lanes past the end re-read the first ref, which changes no box)
+    int b0 = fkey(F_INF), b1 = b0, b2 = b0, b3 = fkey(-F_INF), b4 = b3, b5 = b3;
+    for (int g = 0; g < its; g += G) {
+        load(g);
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            b0 = min(b0, k0[q]); b1 = min(b1, k1[q]); b2 = min(b2, k2[q]);
+            b3 = max(b3, k3[q]); b4 = max(b4, k4[q]); b5 = max(b5, k5[q]);
+        }
+        if (HOLD) break;
+    }
+    const f3 rMin = {unkey(wave_min(b0)), unkey(wave_min(b1)), unkey(wave_min(b2))};
+    const f3 rMax = {unkey(wave_max(b3)), unkey(wave_max(b4)), unkey(wave_max(b5))};
+    int ax;
+    float sp;
+    node_split(rMin, rMax, ax, sp);
+    ax = __builtin_amdgcn_readfirstlane(ax);
+    const int pl = a.empty_space && (d || a.active_index)
+                       ? __builtin_amdgcn_readfirstlane(empty_planes(rMin, rMax, it.mn, it.mx, a.thr))
+                       : 0;
+    auto sides = [&](int g, int q, bool &l, bool &r) {
+        const bool valid = (g + q) * 64 + lane < n;
+        l = valid && unkey(pick3(ax, k0[q], k1[q], k2[q])) <= sp;
+        r = valid && sp < unkey(pick3(ax, k3[q], k4[q], k5[q]));
+    };
+    int cl = 0, cr = 0;
+    for (int g = 0; g < its; g += G) {
+        if (!HOLD) load(g);
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            bool l, r;
+            sides(g, q, l, r);
+            cl += __popcll(__ballot(l));
+            cr += __popcll(__ballot(r));
+        }
+        if (HOLD) break;
+    }
+    const bool leafL = cl < a.LS, leafR = cr < a.LS;
+    const int kids = (leafL ? 0 : 1) + (leafR ? 0 : 1);
+    const int ln = (leafL ? cl : 0) + (leafR ? cr : 0);      // leaf refs
+    const int nL = leafL ? 0 : cl, nR = leafR ? 0 : cr;      // list entries
+    // the children's slots, items and lists, the leaf refs' places
+    int first = 0, at = 0, item = 0, oL = 0;
+    if (lane == 0) {
+        if (kids) {
+            first = atomicAdd(&sh.slots, kids);
+            item = atomicAdd(&sh.cnt[(d & 1) ^ 1], kids);
+            oL = atomicAdd(&sh.used[(d & 1) ^ 1], nL + nR);
+        }
+        if (ln) at = atomicAdd(&sh.leaf, ln);
+    }
+    first = __builtin_amdgcn_readfirstlane(first);
+    item = __builtin_amdgcn_readfirstlane(item);
+    oL = __builtin_amdgcn_readfirstlane(oL);
+    at = __builtin_amdgcn_readfirstlane(at);
+    const int oR = oL + nL, sL = slot0 + first, sR = sL + (leafL ? 0 : 1);
+    bool ok = oR + nR <= SH::entries;
+    if (kids && (first + kids > slot_cap || item + kids > SH::nodes || d + 1 >= SUB_LEVELS)) ok = false;
+    int lb = SUB_GROW * start + at;
+    if (at + ln > SUB_GROW * count) {  // the subtree's places are used up: from the arena
+        if (lane == 0) at = atomicAdd(&a.ctl[1], ln);
+        at = __builtin_amdgcn_readfirstlane(at);
+        const long long b = (long long)SUB_GROW * a.R + at;
+        if (at < 0 || b + ln > a.xcap) ok = false;
+        lb = ok ? (int)b : 0;
+    }
+    if (!ok) {
+        if (lane == 0) sh.fail = 1;
+        return;
+    }
+    const int lbR = lb + (leafL ? cl : 0);
+    const int sk = fkey(sp);
+    const unsigned long long lt = lanemask_lt();
+    int rl = leafL ? lb : oL, rr = leafR ? lbR : oR;
+    for (int g = 0; g < its; g += G) {
+        if (!HOLD) load(g);
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            bool l, r;
+            sides(g, q, l, r);
+            const unsigned long long blm = __ballot(l), brm = __ballot(r);
+            const int dl = rl + __popcll(blm & lt), dr = rr + __popcll(brm & lt);
+            if (l && !leafL) out[dl] = (unsigned short)ix[q];
+            if (r && !leafR) out[dr] = (unsigned short)ix[q];
+            if ((l && leafL) || (r && leafR)) {
+                const float id = a.smin[start + ix[q]].w;
+                const f3 mn = {unkey(k0[q]), unkey(k1[q]), unkey(k2[q])};
+                const f3 mx = {unkey(k3[q]), unkey(k4[q]), unkey(k5[q])};
+                if (l && leafL) {
+                    const float cut = unkey(min(sk, pick3(ax, k3[q], k4[q], k5[q])));
+                    a.xmin[dl] = make_float4(mn.x, mn.y, mn.z, id);
+                    a.xmax[dl] = make_float4(ax == AX_X ? +cut : +mx.x, ax == AX_Y ? +cut : +mx.y,
+                                             ax == AX_Z ? +cut : +mx.z, 0.0f);
+                }
+                if (r && leafR) {
+                    const float cut = unkey(max(sk, pick3(ax, k0[q], k1[q], k2[q])));
+                    a.xmin[dr] = make_float4(ax == AX_X ? +cut : +mn.x, ax == AX_Y ? +cut : +mn.y,
+                                             ax == AX_Z ? +cut : +mn.z, id);
+                    a.xmax[dr] = make_float4(mx.x, mx.y, mx.z, 0.0f);
+                }
+            }
+            rl += __popcll(blm);
+            rr += __popcll(brm);
+        }
+        if (HOLD) break;
+    }
+    if (lane < SUB_COUNTS) {
+        // (a division only where a child is longer than a chunk)
+        const int segs = max(nL, nR) <= a.seg ? kids : (nL + a.seg - 1) / a.seg + (nR + a.seg - 1) / a.seg;
+        const int v = lane == 0 ? 2 * __popc(pl) : lane == 1 ? cl : lane == 2 ? cr : lane == 3 ? (int)leafL
+                    : lane == 4 ? (int)leafR : lane == 5 ? cl - nL : lane == 6 ? cr - nR : segs;
+        atomicAdd(&sh.tot[d * SUB_COUNTS + lane], v);
+    }
+    auto child = [&](bool right) {
+        SubItem c;
+        c.base = right ? oR : oL; c.n = right ? cr : cl;
+        c.slot = right ? sR : sL;
+        c.mn = f3{right && ax == AX_X ? sp : +rMin.x, right && ax == AX_Y ? sp : +rMin.y,
+                  right && ax == AX_Z ? sp : +rMin.z};
+        c.mx = f3{!right && ax == AX_X ? sp : +rMax.x, !right && ax == AX_Y ? sp : +rMax.y,
+                  !right && ax == AX_Z ? sp : +rMax.z};
+        c.c0 = right && ax == AX_X ? max(sk, it.c0) : +it.c0;
+        c.c1 = right && ax == AX_Y ? max(sk, it.c1) : +it.c1;
+        c.c2 = right && ax == AX_Z ? max(sk, it.c2) : +it.c2;
+        c.c3 = !right && ax == AX_X ? min(sk, it.c3) : +it.c3;
+        c.c4 = !right && ax == AX_Y ? min(sk, it.c4) : +it.c4;
+        c.c5 = !right && ax == AX_Z ? min(sk, it.c5) : +it.c5;
+        return c;
+    };
+    if (lane == 0) {
+        int4 *const rec = a.rec + 3ll * it.slot;
+        rec[0] = make_int4(__float_as_int(rMin.x), __float_as_int(rMin.y), __float_as_int(rMin.z), cl);
+        rec[1] = make_int4(__float_as_int(rMax.x), __float_as_int(rMax.y), __float_as_int(rMax.z), cr);
+        rec[2] = make_int4(leafL ? lb : sL, leafR ? lbR : sR, ax, pl);
+        if (!leafL) sub_put(sh, d + 1, item, child(false));
+        if (!leafR) sub_put(sh, d + 1, item + (leafL ? 0 : 1), child(true));
+    }
+}
+
+// node records a subtree may take: SUB_SLOTS per lower_size refs of its root
+// and 32 (every one holds at least lower_size refs)
+constexpr int SUB_SLOTS = 24;
+__host__ __device__ inline long long sub_slot_base(long long first_ref, long long i, int LS) {
+    return SUB_SLOTS * first_ref / LS + 32 * i;
+}
+
+// One block per active node of the level, of those with MIN < refs <= CAP.  The
+// block's waves share out the nodes of a depth and meet before the next.
+template <int MIN, int CAP, int LIST, int NODES, int W>
+__global__ __launch_bounds__(W * 64) void subtree_kernel(NodePtrs N, SubArgs a) {
+    static_assert(CAP <= 65536 && CAP <= LIST, "16-bit indices; the root's own list");
+    __shared__ SubShared<CAP, LIST, NODES> sh;
+    const int t = threadIdx.x, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int i = blockIdx.x, node = a.active_index + i;
+    const int n = (int)N.bitmap[node];
+    if (n > CAP || n <= MIN) {
+        if (n > SUB_MAX && t == 0) atomicOr(&a.ctl[0], 1);
+        return;
+    }
+    const int start = N.prim_index[node];
+    const int slot0 = (int)sub_slot_base(start, i, a.LS);
+    const int slot_cap = (int)(sub_slot_base((long long)start + n, i + 1, a.LS) - slot0);
+    for (int k = t; k < SUB_LEVELS * SUB_COUNTS; k += W * 64) sh.tot[k] = 0;
+    for (int k = t; k < n; k += W * 64) {
+        const float4 mn = a.smin[start + k], mx = a.smax[start + k];
+        sh.key[0][k] = fkey(mn.x); sh.key[1][k] = fkey(mn.y); sh.key[2][k] = fkey(mn.z);
+        sh.key[3][k] = fkey(mx.x); sh.key[4][k] = fkey(mx.y); sh.key[5][k] = fkey(mx.z);
+        sh.list[0][k] = (unsigned short)k;
+    }
+    if (t == 0) {
+        sh.cnt[0] = sh.cnt[1] = sh.used[0] = sh.used[1] = 0;
+        sh.slots = 1; sh.leaf = 0; sh.fail = 0;
+        a.slot[i] = slot0;
+        const float4 mn = N.bmin[node], mx = N.bmax[node];
+        sub_put(sh, 0, 0, SubItem{0, n, slot0, {mn.x, mn.y, mn.z}, {mx.x, mx.y, mx.z}, INT_MIN, INT_MIN, INT_MIN,
+                                  INT_MAX, INT_MAX, INT_MAX});
+    }
+    __syncthreads();
+    int items = 1;
+    for (int d = 0; d < SUB_LEVELS; ++d) {
+        // (the head of this loop is wave-uniform: with the nodes handed out by a
+        // ticket that one lane takes, the compiler joins that branch to the
+        // one-lane branch at the loop's end, and the other lanes go round
+        // without it)
+        for (int k = w; k < items; k += W) {
+            const SubItem it = sub_get(sh, d, k);
+            if (it.n <= 64) sub_node<true, 1>(a, sh, it, d, start, n, slot0, slot_cap);
+            else if (it.n <= 128) sub_node<true, 2>(a, sh, it, d, start, n, slot0, slot_cap);
+            else sub_node<false, 2>(a, sh, it, d, start, n, slot0, slot_cap);
+            __builtin_amdgcn_wave_barrier();
+        }
+        __syncthreads();
+        // between the barriers nothing writes what every wave reads here
+        items = __builtin_amdgcn_readfirstlane(sh.cnt[(d & 1) ^ 1]);
+        const int failed = __builtin_amdgcn_readfirstlane(sh.fail);
+        if (t == 0) sh.cnt[d & 1] = sh.used[d & 1] = 0;
+        __syncthreads();
+        if (failed || items == 0) break;
+    }
+    int *const tot = a.tot + (long long)(i % SUB_COPIES) * SUB_LEVELS * SUB_COUNTS;
+    for (int k = t; k < SUB_LEVELS * SUB_COUNTS; k += W * 64)
+        if (sh.tot[k]) atomicAdd(&tot[k], sh.tot[k]);
+    if (t == 0 && sh.fail) atomicOr(&a.ctl[0], 1);
+}
+
+// the levels' totals and the failure flag to the host, tagged with seq; both
+// cleared for the next build
+__global__ __launch_bounds__(SUB_WORDS) void sub_publish_kernel(int *__restrict__ tot, int *__restrict__ ctl,
+                                                                unsigned long long *host, unsigned seq) {
+    const int t = threadIdx.x;
+    int v = 0;
+    if (t < SUB_WORDS - 1) {
+#pragma unroll 16
+        for (int r = 0; r < SUB_COPIES; ++r) v += tot[r * (SUB_WORDS - 1) + t];
+        for (int r = 0; r < SUB_COPIES; ++r) tot[r * (SUB_WORDS - 1) + t] = 0;
+    } else {
+        v = ctl[0];
+        ctl[0] = 0;
+        ctl[1] = 0;
+    }
+    __hip_atomic_store(&host[t], (unsigned long long)seq << 32 | (unsigned)v, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// A level of the subtrees: its plan (known from the totals) and buffers.
+struct NumArgs {
+    int A, active_index, child_start, next_active, leaf_nodes, leaf_left, L_all, LL_all, ulp, nleaf, nleaf0;
+    int LS, propagate, par, depth;
+    const int4 *rec;
+    const int *slot;
+    int *slot_n;
+    int4 *mv;                          // per leaf from nleaf0 on: first ref, destination, refs
+    unsigned long long *lb, *lb_n;
+    int *ctr;
+};
+
+// The nodes of a level, one per thread: the scans, chains and child records
+// the leaf and scatter passes make.  Everything of the level is written in this
+// one launch, since the totals that number the right children are known.
+__global__ __launch_bounds__(LBS) void number_pass_kernel(NodePtrs N, Lvl *L, NumArgs P,
+                                                         int *__restrict__ leaf_ids) {
+    __shared__ int s_tile;
+    __shared__ int s_w[7][LBS / 64];
+    __shared__ long long s_ex[7];
+    const int t = threadIdx.x;
+    if (t == 0) {
+        s_tile = atomicAdd(&P.ctr[P.par], 1);
+    }
+    __syncthreads();
+    const int tile = s_tile;           // (as many blocks as tiles)
+    const int i = tile * LBS + t, node = P.active_index + i;
+    const bool in_tile = i < P.A;
+    int4 r0 = make_int4(0, 0, 0, 0), r1 = r0, r2 = r0;
+    int parent = 0;
+    bool left = false;
+    int v[7] = {0, 0, 0, 0, 0, 0, 0};
+    if (in_tile) {
+        const int4 *rec = P.rec + 3ll * P.slot[i];
+        parent = N.parent[node];
+        r0 = rec[0]; r1 = rec[1]; r2 = rec[2];
+        left = N.children[parent].x == node;
+        const bool lL = r0.w < P.LS, lR = r1.w < P.LS;
+        v[0] = r0.w; v[1] = r1.w; v[2] = 2 * __popc(r2.w);
+        v[3] = lL; v[4] = lR; v[5] = lL ? r0.w : 0; v[6] = lR ? r1.w : 0;
+    }
+    int pre[7], tot[7];
+    block_scan<7, LBS>(v, pre, tot, s_w);
+    if (t < 64) {
+        const long long agg[7] = {tot[0], tot[1], tot[2], tot[3], tot[4], tot[5], tot[6]};
+        long long ex[7];
+        lookback<7>(P.lb, tile, agg, ex, &L->status);
+        if (t == 0)
+            for (int k = 0; k < 7; ++k) s_ex[k] = ex[k];
+    }
+    __syncthreads();
+    if (in_tile) {
+        const f3 rMin = {__int_as_float(r0.x), __int_as_float(r0.y), __int_as_float(r0.z)};
+        const f3 rMax = {__int_as_float(r1.x), __int_as_float(r1.y), __int_as_float(r1.z)};
+        int ax;
+        float sp;
+        node_split(rMin, rMax, ax, sp);
+        N.bmin[node] = make_float4(rMin.x, rMin.y, rMin.z, 0.0f);
+        N.bmax[node] = make_float4(rMax.x, rMax.y, rMax.z, 0.0f);
+        N.split[node] = sp;
+        N.info[node] = (int8_t)ax;
+        if (r2.w)
+            empty_chain_node_at(N, node, P.active_index + P.A + (int)s_ex[2] + pre[2], r2.w, parent, left, rMin, rMax);
+        const int sizes[2] = {r0.w, r1.w};
+        const int kid[2] = {r2.x, r2.y};
+        const bool leaf[2] = {sizes[0] < P.LS, sizes[1] < P.LS};
+        const int lna[2] = {(int)s_ex[3] + pre[3], P.leaf_left + (int)s_ex[4] + pre[4]};
+        const int leaf_addr[2] = {(int)s_ex[5] + pre[5], P.LL_all + (int)s_ex[6] + pre[6]};
+        const int split_addr[2] = {(int)s_ex[0] + pre[0], P.L_all + (int)s_ex[1] + pre[1]};
+        int ids[2];
+#pragma unroll
+        for (int side = 0; side < 2; ++side) {
+            const int id = P.child_start + (leaf[side] ? lna[side] : side * P.A + i - lna[side] + P.leaf_nodes);
+            ids[side] = id;
+            const int at = leaf[side] ? leaf_addr[side] + P.ulp : split_addr[side] - leaf_addr[side];
+            N.prim_index[id] = at;
+            N.bitmap[id] = sizes[side];
+            N.area[id] = 0.0f;
+            N.parent[id] = node;
+            if (leaf[side]) {
+                N.info[id] = LEAF; N.split[id] = 0.0f;
+                N.children[id] = make_int2(0, 0);
+                float4 mn = make_float4(0.0f, 0.0f, 0.0f, 0.0f), mx = mn;
+                if (P.propagate) {
+                    mn = make_float4(rMin.x, rMin.y, rMin.z, 0.0f);
+                    mx = make_float4(rMax.x, rMax.y, rMax.z, 0.0f);
+                    float4 &cut = side ? mn : mx;
+                    cut.x = ax == AX_X ? sp : cut.x; cut.y = ax == AX_Y ? sp : cut.y; cut.z = ax == AX_Z ? sp : cut.z;
+                }
+                N.bmin[id] = mn;
+                N.bmax[id] = mx;
+                leaf_ids[P.nleaf + lna[side]] = id;
+                P.mv[P.nleaf - P.nleaf0 + lna[side]] = make_int4(kid[side], at, sizes[side], 0);
+            } else {
+                // (the child's own tile of the next level writes the rest)
+                P.slot_n[id - P.next_active] = kid[side];
+            }
+        }
+        N.children[node] = make_int2(ids[0], ids[1]);
+    }
+    // the next level's status words and ticket
+    const int created = 2 * P.A - P.leaf_nodes;
+    const int words = 8 * max(1, (created + LBS - 1) / LBS);
+    for (int k = blockIdx.x * LBS + t; k < words; k += gridDim.x * LBS) P.lb_n[k] = 0ull;
+    if (blockIdx.x == 0 && t == 0) P.ctr[P.par ^ 1] = 0;
+}
+
+// The subtrees' leaf refs to their places, 16 lanes a leaf; the level state
+// after the last level.
+constexpr int MOVE_LANES = 16;
+__global__ __launch_bounds__(BS) void leaf_move_kernel(Lvl *L, Lvl v, const int4 *__restrict__ mv, int n,
+                                                       const float4 *__restrict__ xmin,
+                                                       const float4 *__restrict__ xmax, float4 *__restrict__ fmin,
+                                                       float4 *__restrict__ fmax) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (L->status) lvl_fail(&v, L->status);   // a look-back that failed
+        *L = v;
+    }
+    const int lane = threadIdx.x % MOVE_LANES;
+    for (int k = (blockIdx.x * BS + threadIdx.x) / MOVE_LANES; k < n; k += gridDim.x * BS / MOVE_LANES) {
+        const int4 m = mv[k];
+        for (int j = lane; j < m.z; j += MOVE_LANES) {
+            const float4 a = xmin[m.x + j], b = xmax[m.x + j];
+            fmin[m.y + j] = a;
+            fmax[m.y + j] = b;
+        }
+    }
 }
 
 // PropagateParentAabb<true> (EmptySpaceSplitting.h:333-368)
@@ -2311,7 +2809,7 @@ __global__ void build_init_kernel(Lvl *L, Lvl v, NodePtrs N, const int *__restri
         lb0[k] = 0ull;
         lb1[k] = 0ull;
     }
-    if (blockIdx.x == 0 && threadIdx.x < 2) ctr[threadIdx.x] = 0;
+    if (blockIdx.x == 0 && threadIdx.x < 4) ctr[threadIdx.x] = 0;
 }
 
 // a captured build that needed more levels than it recorded
@@ -2331,14 +2829,12 @@ void read_state(BuildScratch &sc, Lvl &h, hipStream_t s) {
 // an eager level's state as its leaf pass published it (sequence number
 // seq); the stream is queried now and then, so a pass that failed to run
 // reports the stream's error instead of being waited for
-void wait_level(BuildScratch &sc, Lvl &h, unsigned seq, hipStream_t s) {
-    const LvlMirror::Rec *m = sc.mirror.host + (seq & 1u);
-    int words[LvlMirror::NW];
-    // every word of the record tagged with seq (word 0 is the cheap spin)
+void wait_words(const unsigned long long *m, int *words, int n, unsigned seq, hipStream_t s) {
+    // every word tagged with seq (word 0 is the cheap spin)
     auto take = [&]() {
-        if ((unsigned)(__atomic_load_n(&m->w[0], __ATOMIC_ACQUIRE) >> 32) != seq) return false;
-        for (int t = 0; t < LvlMirror::NW; ++t) {
-            const unsigned long long v = __atomic_load_n(&m->w[t], __ATOMIC_ACQUIRE);
+        if ((unsigned)(__atomic_load_n(&m[0], __ATOMIC_ACQUIRE) >> 32) != seq) return false;
+        for (int t = 0; t < n; ++t) {
+            const unsigned long long v = __atomic_load_n(&m[t], __ATOMIC_ACQUIRE);
             if ((unsigned)(v >> 32) != seq) return false;
             words[t] = (int)(unsigned)v;
         }
@@ -2352,6 +2848,11 @@ void wait_level(BuildScratch &sc, Lvl &h, unsigned seq, hipStream_t s) {
         if (take()) break;
         throw Error{PM_ERR_INTERNAL, "a level's state was not published"};
     }
+}
+
+void wait_level(BuildScratch &sc, Lvl &h, unsigned seq, hipStream_t s) {
+    int words[LvlMirror::NW];
+    wait_words(sc.mirror.host[seq & 1u].w, words, LvlMirror::NW, seq, s);
     std::memcpy(&h, words, sizeof(Lvl));
 }
 
@@ -2382,6 +2883,8 @@ inline int grid_for(long long n, int per, int cap) {
 // bound)
 constexpr long long AHEAD_REFS = 1 << 17;
 constexpr long long AHEAD_NODES = 1 << 14;   // the same for the nodes of a lower level
+constexpr long long SUB_REFS = 1 << 17;      // triangles of a build up to which its nodes go to subtrees (subtree_kernel),
+                                             // while a level has at most twice as many refs
 
 // the sizes of a level (exact, or bounds of them): active nodes, refs,
 // segments, and the nodes, leaf refs and leaf ids written before it
@@ -2414,6 +2917,125 @@ void reserve_first(pm_ctx *ctx, int N, int M, int seg, hipStream_t s) {
     sc.prim_min.reserve((size_t)r + 1, s); sc.prim_max.reserve((size_t)r + 1, s);
     ctx->leaf_ids.reserve((size_t)n / 2 + 2 * M, s);
     ctx->nodes.reserve((size_t)(n + n / 2) + 1024 + 16 * M, s, 0);
+}
+
+// The upper stage's remaining levels by the subtrees of level `par`'s nodes (see
+// subtree_kernel).  h: the level state with that level's advance to come; on
+// success the state after the last level (on the device too).  false, and
+// nothing changed, when the subtrees cannot hold the build: the level loop
+// goes on and reports what there is to report.
+bool build_subtrees(pm_ctx *ctx, Lvl &h, int par, int S, int max_n, const pm_build_params &prm, int seg,
+                    BuildSizes &seen, hipStream_t s) {
+    BuildScratch &sc = ctx->scratch;
+    const int nxt = par ^ 1, LS = prm.lower_size;
+    Lvl g = h;
+    advance_level(&g);
+    const long long A = g.A, R = g.R, slots = sub_slot_base(R, A + 1, LS);
+    if (g.status || A == 0 || slots > INT_MAX / 4) return false;
+    const long long xcap = (SUB_GROW + SUB_ARENA) * R;
+    sc.ref_min[nxt].reserve((size_t)xcap + 1, s); sc.ref_max[nxt].reserve((size_t)xcap + 1, s);
+    sc.sub_rec.reserve(3 * (size_t)slots, s);
+    sc.sub_slot[0].reserve((size_t)A + 1, s);
+    constexpr int TOT = SUB_COPIES * SUB_LEVELS * SUB_COUNTS;
+    if (!sc.sub_tot.ptr) {
+        sc.sub_tot.reserve(TOT + 2, s);
+        PM_HIP(hipMemsetAsync(sc.sub_tot.ptr, 0, (TOT + 2) * sizeof(int), s));
+    }
+    SubArgs a{};
+    a.smin = sc.ref_min[par].ptr; a.smax = sc.ref_max[par].ptr;
+    a.xmin = sc.ref_min[nxt].ptr; a.xmax = sc.ref_max[nxt].ptr;
+    a.xcap = xcap;
+    a.rec = sc.sub_rec.ptr;
+    a.slot = sc.sub_slot[0].ptr;
+    a.tot = sc.sub_tot.ptr; a.ctl = sc.sub_tot.ptr + TOT;
+    a.active_index = g.active_index; a.R = (int)R; a.LS = LS; a.seg = seg;
+    a.empty_space = prm.empty_space_splitting;
+    a.thr = prm.empty_space_threshold;
+    if (max_n > SUB_SMALL) {
+        subtree_kernel<SUB_SMALL, SUB_MAX, 4 * SUB_MAX, 96, 16><<<(int)A, 16 * 64, 0, s>>>(node_ptrs(ctx), a);
+        PM_LAUNCH_CHECK();
+    }
+    subtree_kernel<-1, SUB_SMALL, 4 * SUB_SMALL, 48, 8><<<(int)A, 8 * 64, 0, s>>>(node_ptrs(ctx), a);
+    PM_LAUNCH_CHECK();
+    const unsigned seq = sc.mirror.take_seq();
+    sub_publish_kernel<<<1, SUB_WORDS, 0, s>>>(a.tot, a.ctl, sc.mirror.sub_dev, seq);
+    PM_LAUNCH_CHECK();
+    int tot[SUB_WORDS];
+    wait_words(sc.mirror.sub_host, tot, SUB_WORDS, seq, s);
+    if (tot[SUB_WORDS - 1]) return false;
+
+    // the levels' plans from their totals, as the leaf pass's last tile makes them
+    std::vector<NumArgs> plans;
+    std::vector<long long> level_refs;
+    BuildSizes sn = seen;
+    const int nleaf0 = g.nleaf;
+    long long max_A = 0;
+    for (int d = 0; g.A > 0; ++d) {
+        if (d >= SUB_LEVELS) return false;
+        const int *const c = tot + d * SUB_COUNTS;
+        const long long newTri = (long long)c[1] + c[2];
+        NumArgs P{};
+        P.A = g.A; P.active_index = g.active_index; P.ulp = g.final_refs; P.nleaf = g.nleaf; P.nleaf0 = nleaf0;
+        g.E = c[0];
+        g.S = S;
+        g.nodes_size += c[0];
+        g.seen_active = std::max<long long>(g.seen_active, g.A);
+        g.seen_segs = std::max<long long>(g.seen_segs, S);
+        g.seen_refs = std::max<long long>(g.seen_refs, g.R);
+        g.L_all = c[1]; g.R_all = c[2]; g.LL_all = c[5]; g.LR_all = c[6];
+        g.leaf_left = c[3];
+        g.leaf_nodes = c[3] + c[4];
+        g.leafTri = c[5] + c[6];
+        g.nextR = (int)(newTri - g.leafTri);
+        g.created = 2 * g.A - g.leaf_nodes;
+        g.child_start = g.nodes_size;
+        g.next_active = g.nodes_size + g.leaf_nodes;
+        if (newTri < g.R || newTri > INT_MAX || (g.created > 0 && g.nextR > g.max_refs)) return false;
+        P.child_start = g.child_start; P.next_active = g.next_active;
+        P.leaf_nodes = g.leaf_nodes; P.leaf_left = g.leaf_left; P.L_all = g.L_all; P.LL_all = g.LL_all;
+        P.LS = LS; P.propagate = prm.empty_space_splitting; P.par = (par + d) & 1; P.depth = d;
+        plans.push_back(P);
+        level_refs.push_back(g.R);
+        sn.refs = std::max<long long>(sn.refs, g.R);
+        sn.active = std::max<long long>(sn.active, g.A);
+        sn.segs = std::max<long long>({sn.segs, (long long)S, (long long)c[7]});
+        max_A = std::max<long long>(max_A, g.A);
+        S = c[7];
+        g.advance = 1;
+        advance_level(&g);
+        if (g.status) return false;
+    }
+
+    const int moved = g.nleaf - nleaf0;
+    ctx->nodes.reserve((size_t)g.nodes_size + 1, s, (size_t)plans[0].child_start);
+    sc.prim_min.reserve((size_t)g.final_refs + 1, s, (size_t)plans[0].ulp);
+    sc.prim_max.reserve((size_t)g.final_refs + 1, s, (size_t)plans[0].ulp);
+    ctx->leaf_ids.reserve((size_t)g.nleaf + 1, s, (size_t)nleaf0);
+    sc.sub_move.reserve((size_t)moved + 1, s);
+    sc.sub_slot[0].reserve((size_t)max_A + 1, s, (size_t)A);
+    sc.sub_slot[1].reserve((size_t)max_A + 1, s);
+    const long long words = 8 * ((max_A + LBS - 1) / LBS) + 8;
+    sc.lb_words[par].reserve((size_t)words, s, 8 * (size_t)((A + LBS - 1) / LBS));
+    sc.lb_words[nxt].reserve((size_t)words, s);
+    const NodePtrs NP = node_ptrs(ctx);
+    for (NumArgs &P : plans) {
+        P.rec = sc.sub_rec.ptr;
+        P.slot = sc.sub_slot[P.depth & 1].ptr;
+        P.slot_n = sc.sub_slot[(P.depth & 1) ^ 1].ptr;
+        P.mv = sc.sub_move.ptr;
+        P.lb = sc.lb_words[P.par].ptr; P.lb_n = sc.lb_words[P.par ^ 1].ptr;
+        P.ctr = sc.lb_ctr.ptr;
+        number_pass_kernel<<<blocks_for(P.A, LBS), LBS, 0, s>>>(NP, sc.lvl.ptr, P, ctx->leaf_ids.ptr);
+        PM_LAUNCH_CHECK();
+    }
+    leaf_move_kernel<<<grid_for((long long)moved * MOVE_LANES, BS, 1 << 16), BS, 0, s>>>(
+        sc.lvl.ptr, g, sc.sub_move.ptr, moved, a.xmin, a.xmax, sc.prim_min.ptr,
+        sc.prim_max.ptr);
+    PM_LAUNCH_CHECK();
+    ctx->level_refs.insert(ctx->level_refs.end(), level_refs.begin(), level_refs.end());
+    seen = sn;
+    h = g;
+    return true;
 }
 
 // The build's kernel sequence.  caps == nullptr: eager (each upper level's
@@ -2530,10 +3152,22 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
     // take longer, 650 -> 637).  The build ends after the level that creates no active node; a
     // level launched past it has no nodes and writes none.
     LevelSizes known{M, N, S_now, M, 0, 0};   // the level after the last one whose state is known
+    int known_max = 0;                        // the largest node of the known level
+    // the subtrees of a small build's level whose nodes hold up to SUB_MAX refs (a captured
+    // batch keeps its buffers, and the DIVIDE split its own passes; with small
+    // leaves the straddling refs outgrow a subtree's room)
+    bool subtrees = run_ahead && !div && LS >= 16 && N <= SUB_REFS;
+    auto to_subtrees = [&]() { return subtrees && known_max <= SUB_MAX && known.R <= 2 * SUB_REFS; };
+    for (int m = 0; subtrees && m < M; ++m)
+        known_max = std::max(known_max, ctx->mesh_offsets[m + 1] - ctx->mesh_offsets[m]);
     std::deque<unsigned> out;                 // levels launched after that, not taken yet
     bool done = false;
     for (int lvl = 0; graph ? lvl < caps->upper_levels : !done; ++lvl) {
         const int par = lvl & 1, nxt = par ^ 1;
+        if (out.empty() && to_subtrees()) {
+            if (build_subtrees(ctx, h, par, (int)known.S, known_max, prm, seg, seen, s)) break;
+            subtrees = false;
+        }
         LevelSizes b = known;
         for (size_t k = 0; k < out.size(); ++k) b = b.next_bound(seg);
         const long long A_now = b.A;
@@ -2566,9 +3200,13 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
                                                                 ? grid_for(12 * KEY_REPL * A_g, 4 * LBS, 2048)
                                                                 : grid_for(12 * A_g, 16 * BS, 2048));
         const unsigned seq = mirror ? sc.mirror.take_seq() : 0u;
-        leaf_pass_kernel<<<graph ? std::min(g3, 2048) : g3, LBS, 0, s>>>(
-            NP, L, B, par, LS, seg, sc.keys[par].ptr, sc.keys[nxt].ptr, prm.empty_space_splitting,
-            prm.empty_space_threshold, mirror ? sc.mirror.dev + (seq & 1u) : nullptr, seq);
+        auto leaf_pass = [&](auto kernel) {
+            kernel<<<graph ? std::min(g3, 2048) : g3, LBS, 0, s>>>(
+                NP, L, B, par, LS, seg, sc.keys[par].ptr, sc.keys[nxt].ptr, prm.empty_space_splitting,
+                prm.empty_space_threshold, mirror ? sc.mirror.dev + (seq & 1u) : nullptr, seq);
+        };
+        if (subtrees) leaf_pass(leaf_pass_kernel<true>);
+        else leaf_pass(leaf_pass_kernel<false>);
         PM_LAUNCH_CHECK();
         const int g4 = std::max(grid_for(S_g, WPB, INT_MAX), grid_for(A_g, BS, INT_MAX));
         launch_scatter_pass(seg, div, graph ? std::min(g4, 2048) : g4, s, NP, (const Lvl *)L, B, LS, seg,
@@ -2578,8 +3216,10 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
         PM_LAUNCH_CHECK();
         if (graph) continue;
         out.push_back(seq);
-        const size_t ahead = run_ahead && known.R <= AHEAD_REFS ? 1 : 0;
-        while (out.size() > ahead && !done) {
+        auto ahead = [&]() {   // (a level whose nodes go to subtrees is not launched)
+            return run_ahead && known.R <= AHEAD_REFS && !to_subtrees() ? 1u : 0u;
+        };
+        while (!done && out.size() > ahead()) {
             const int taken = (lvl + 1 - (int)out.size()) & 1;   // the taken level's parity
             if (mirror) wait_level(sc, h, out.front(), s);
             else read_state(sc, h, s);
@@ -2595,6 +3235,7 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
             Lvl n = h;
             advance_level(&n);
             known = LevelSizes{n.A, n.R, h.scanS[taken ^ 1], n.nodes_size, n.final_refs, n.nleaf};
+            known_max = (int)h.max_child;
         }
     }
     // the last level's advance

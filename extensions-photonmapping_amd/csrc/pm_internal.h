@@ -134,7 +134,12 @@ struct Lvl {
     int max_levels;
     long long max_refs;
     long long cap_nodes, cap_active, cap_segs, cap_refs, cap_leaf_refs, cap_leaf_ids, cap_lower;
+    long long max_child;                               // refs of the largest non-leaf child (if looked at)
 };
+
+// The subtrees of an upper level: counts per level below it, and the words of
+// the record the host takes (the counts and a failure flag).
+constexpr int SUB_LEVELS = 48, SUB_COUNTS = 8, SUB_WORDS = SUB_LEVELS * SUB_COUNTS + 1;
 
 // A copy of the level state in coherent pinned host memory: an eager build's
 // upper levels (the last tile of the leaf pass) and lower levels (the plan
@@ -152,6 +157,8 @@ struct LvlMirror {
     };
     Rec *host = nullptr;   // coherent, mapped: two records, a level's is [number & 1]
     Rec *dev = nullptr;    // the device's address of them
+    // after them: the subtrees' counts, tagged the same way
+    unsigned long long *sub_host = nullptr, *sub_dev = nullptr;
     unsigned next_seq = 0;
     // the next level's number: odd and even in turn (a level launched before
     // the one before it is taken writes the other record), never 0, the tag
@@ -172,7 +179,8 @@ struct LvlMirror {
             failed = true;
             return false;
         }
-        if (hipHostMalloc((void **)&host, 2 * sizeof(Rec), hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess ||
+        const size_t bytes = 2 * sizeof(Rec) + SUB_WORDS * sizeof(unsigned long long);
+        if (hipHostMalloc((void **)&host, bytes, hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess ||
             hipHostGetDevicePointer((void **)&dev, host, 0) != hipSuccess) {
             (void)hipGetLastError();
             if (host) (void)hipHostFree(host);
@@ -181,7 +189,10 @@ struct LvlMirror {
             failed = true;
             return false;
         }
+        sub_host = reinterpret_cast<unsigned long long *>(host + 2);
+        sub_dev = reinterpret_cast<unsigned long long *>(dev + 2);
         for (int t = 0; t < 2 * NW; ++t) __atomic_store_n(&host[t / NW].w[t % NW], 0ull, __ATOMIC_RELEASE);
+        for (int t = 0; t < SUB_WORDS; ++t) __atomic_store_n(&sub_host[t], 0ull, __ATOMIC_RELEASE);
         return true;
     }
 };
@@ -205,6 +216,8 @@ struct BuildScratch {
     DevBuf<int4> node_rec;                      // per active node: 3 records for the scatter pass (LevelBufs::rec)
     DevBuf<unsigned long long> lb_words[2];     // look-back status words of the leaf passes (by level parity)
     DevBuf<int> lb_ctr;                         // their tile tickets (by level parity)
+    DevBuf<int4> sub_rec, sub_move;             // subtrees: node records, leaf refs to move
+    DevBuf<int> sub_slot[2], sub_tot;           // subtrees: active nodes' records (by level parity), counts per level
     DevBuf<int> scan_tmp[3];                    // block sums for scans, per level
     DevBuf<int> totals;                         // small device-side counters
     DevBuf<unsigned long long> prims_part;      // lower stage: prims counted per wave slot (64)
