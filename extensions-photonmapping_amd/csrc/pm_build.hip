@@ -2471,6 +2471,45 @@ __global__ __launch_bounds__(WPB * 64) void sah_kernel(
     }
 }
 
+// Screen and search in one launch, a wave a node, for levels of up to
+// LOWER_SMALL nodes where nodes are forced to split: most of them are searched,
+// and either pass takes the time of one node's chain (5 to 6 us) and its launch.
+// A 5,316-triangle room with 8 lower levels of up to 2,334 nodes 574 -> 536 us.
+// Without forced splits the screen settles most nodes lane by lane, and a wave
+// for each costs more (soups of 2,000 triangles 262 -> 281 us); larger levels
+// keep their waves for the nodes that need the search.
+constexpr int LOWER_SMALL = 4096;
+__global__ __launch_bounds__(WPB * 64) void sah_level_kernel(
+    NodePtrs N, const int *__restrict__ leaf_ids, const Lvl *__restrict__ L, const float4 *__restrict__ pmin,
+    const float4 *__restrict__ pmax, const float *__restrict__ areas, float Ct, int leaf_max, float bonus,
+    int *__restrict__ flag, long long *__restrict__ sets, float *__restrict__ careas,
+    unsigned long long *__restrict__ parts) {
+    __shared__ SahLds lds;
+    const int An = L->An, list_base = L->list_base;
+    const int *list = L->use_list ? leaf_ids : nullptr;
+    const int lane = threadIdx.x & 63;
+    for (int id = __builtin_amdgcn_readfirstlane(wave_index()); id < An; id += wave_count()) {
+        const int par = __builtin_amdgcn_readfirstlane(list ? list[id] : list_base + id);
+        const unsigned long long bmp = lane_u64((unsigned long long)N.bitmap[par], 0);
+        const float nodeA = lane_float(N.area[par], 0);
+        const int pi = __builtin_amdgcn_readfirstlane(N.prim_index[par]);
+        const int n = __popcll(bmp);
+        const float leaf_cost = ((float)n - Ct) * nodeA;
+        bool search = leaf_max > 0 && n > leaf_max;
+        if (!search && leaf_cost > 0.0f)
+            search = !sah_cannot_split(bmp, (bmp >> lane) & 1ull ? areas[pi + lane] : 0.0f, n, bonus, leaf_cost);
+        if (search) sah_node(N, id, par, lds, pmin, pmax, areas, Ct, leaf_max, bonus, flag, sets, careas);
+        if (lane == 0) {
+            atomicAdd(&parts[wave_index() % PRIM_SLOTS], (unsigned long long)n);
+            if (!search) {
+                N.info[par] = LEAF;
+                flag[id] = 0;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();   // (the lanes stay together into the next node)
+    }
+}
+
 // The balanced ("SSAH") creator's decision (CalcSplit with
 // CalcRelationForSets, LowerTriangleMap.h:266-369), one wave per node: the
 // SAH's candidate planes and masks (ballots), cost small^2 + large^2 of the
@@ -3289,7 +3328,12 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
                 balanced_kernel<<<grid_for(nAn, WPB, graph ? 2048 : INT_MAX), WPB * 64, 0, s>>>(
                     NP, ctx->leaf_ids.ptr, L, sc.prim_min.ptr, sc.prim_max.ptr, prm.traversal_cost, LS,
                     sc.lower_flag.ptr, sc.lower_sets.ptr, sc.lower_careas.ptr);
-            else {
+            else if (prm.sah_leaf_max > 0 && nAn <= LOWER_SMALL) {
+                sah_level_kernel<<<grid_for(nAn, WPB, INT_MAX), WPB * 64, 0, s>>>(
+                    NP, ctx->leaf_ids.ptr, L, sc.prim_min.ptr, sc.prim_max.ptr, sc.areas.ptr, prm.traversal_cost,
+                    prm.sah_leaf_max, prm.sah_empty_bonus, sc.lower_flag.ptr, sc.lower_sets.ptr, sc.lower_careas.ptr,
+                    sc.prims_part.ptr);
+            } else {
                 const int npw = screen_nodes(nAn);
                 sah_screen_kernel<<<grid_for((nAn + npw - 1) / npw, WPB, graph ? 1024 : INT_MAX), WPB * 64, 0, s>>>(
                     NP, ctx->leaf_ids.ptr, L, sc.areas.ptr, prm.traversal_cost, prm.sah_leaf_max,
