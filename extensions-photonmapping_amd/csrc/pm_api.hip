@@ -558,7 +558,7 @@ int pm_photon_bounce(pm_ctx *ctx, const float *org, const float *dir, const pm_h
         if (!ctx->p0 && ctx->ntris > 0) throw Error{PM_ERR_NO_TREE, "no geometry"};
         if (absorb_from < 0 || absorb_from > ctx->ntris)
             throw Error{PM_ERR_ARG, "absorb_from must be in [0, triangles of the geometry]"};
-        // the compaction's scan scratch is shared with a captured batch
+        // the compaction's scratch is the context's, which a captured batch uses too
         pmkd::sync_graph_state(ctx, (hipStream_t)stream);
         const int c = pmkd::photon_bounce(ctx, reinterpret_cast<const float4 *>(org),
                                           reinterpret_cast<const float4 *>(dir), hits, n, absorb_from,

@@ -226,7 +226,7 @@ struct BuildScratch {
     DevBuf<int> lower_flag, lower_off;
     DevBuf<long long> lower_sets;               // 2 per node
     DevBuf<float> lower_careas;                 // 2 per node
-    DevBuf<int> bounce_flags, bounce_offs;      // photon driver compaction
+    DevBuf<int> bounce_counts;                  // photon driver compaction: survivors per wave, then all
     DevBuf<float> light_cdf;                    // photon emission: running sum of the light areas
     DevBuf<unsigned> bwd_keys[2], bwd_vals[2];  // backward: radix sort ping-pong
     DevBuf<float> bwd_corner;                   // backward: 3 float3 per ray
