@@ -383,9 +383,9 @@ int pm_trace_noalloc(pm_ctx *ctx, int algo, const float *org, const float *dir, 
         } else if (!ctx->has_tree) {
             throw Error{PM_ERR_NO_TREE, "no tree: call pm_build or pm_set_tree first"};
         }
-        const pmkd::StaticScratch &ss = pmkd::static_scratch(ctx->device);
+        int *const work = pmkd::static_work(ctx->device);
         pmkd::trace_rays(ctx, algo, reinterpret_cast<const float4 *>(org), reinterpret_cast<const float4 *>(dir),
-                         nrays, nullptr, out, prm, reinterpret_cast<int4 *>(counters), (hipStream_t)stream, &ss);
+                         nrays, nullptr, out, prm, reinterpret_cast<int4 *>(counters), (hipStream_t)stream, work);
     });
 }
 

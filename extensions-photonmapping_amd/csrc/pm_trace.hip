@@ -1346,6 +1346,7 @@ void dispatch(const TreeDev &T, int algo, const RayBatch &R, int S, pm_hit *out,
 // 1.9M 1021/962; over 64 (0.9M slots) 0.5M 303/388.
 constexpr int ORDER_PAYS_RAYS = 7 << 18;
 constexpr long long ORDER_PAYS_SLOTS = 1 << 19;
+static_assert(NOALLOC_MAX_ORDERED_RAYS < ORDER_PAYS_RAYS, "the allocation-free trace has no sort buffers");
 bool order_pays(const TreeDev &T, int nrays) { return nrays >= ORDER_PAYS_RAYS && T.num_slots >= ORDER_PAYS_SLOTS; }
 
 template <bool WOOP>
@@ -1520,7 +1521,7 @@ void launch_canvas(bool skip, bool woop, int blocks, hipStream_t s, const TreeDe
 
 void trace_rays(pm_ctx *ctx, int algo, const float4 *org, const float4 *dir, int nrays,
                 const int *ray_mesh, pm_hit *out, const pm_trace_params &prm, int4 *counters,
-                hipStream_t s, const StaticScratch *ext) {
+                hipStream_t s, int *ext_work) {
     if (nrays == 0) return;
     const bool woop = prm.intersection == PM_INTERSECT_WOOP;
     if (algo == PM_TRACE_BRUTE) {
@@ -1548,12 +1549,10 @@ void trace_rays(pm_ctx *ctx, int algo, const float4 *org, const float4 *dir, int
     const int S = prm.stack_size;
     RayBatch R{org, dir, ray_mesh, nullptr, nrays};
     if (ray_order_applies(prm, nrays) && order_pays(T, nrays))
-        R.order = ray_order(ctx, org, dir, ray_mesh, nrays, s, ext ? &ext->order : nullptr);
+        R.order = ray_order(ctx, org, dir, ray_mesh, nrays, s);
     query_cus(ctx);
-    int *work = nullptr;
-    if (ext) {
-        work = ext->work;
-    } else {
+    int *work = ext_work;
+    if (!work) {
         ctx->scratch.trace_work.reserve(1, s);
         work = ctx->scratch.trace_work.ptr;
     }
