@@ -3007,7 +3007,9 @@ bool build_subtrees(pm_ctx *ctx, Lvl &h, int par, int S, int max_n, const pm_bui
     std::vector<NumArgs> plans;
     std::vector<long long> level_refs;
     BuildSizes sn = seen;
-    const int nleaf0 = g.nleaf;
+    // what the levels before have written (and so what growth keeps; the first
+    // level's empty-space nodes are not among it, and need not have had room)
+    const int nodes0 = g.nodes_size, ulp0 = g.final_refs, nleaf0 = g.nleaf;
     long long max_A = 0;
     for (int d = 0; g.A > 0; ++d) {
         if (d >= SUB_LEVELS) return false;
@@ -3046,9 +3048,9 @@ bool build_subtrees(pm_ctx *ctx, Lvl &h, int par, int S, int max_n, const pm_bui
     }
 
     const int moved = g.nleaf - nleaf0;
-    ctx->nodes.reserve((size_t)g.nodes_size + 1, s, (size_t)plans[0].child_start);
-    sc.prim_min.reserve((size_t)g.final_refs + 1, s, (size_t)plans[0].ulp);
-    sc.prim_max.reserve((size_t)g.final_refs + 1, s, (size_t)plans[0].ulp);
+    ctx->nodes.reserve((size_t)g.nodes_size + 1, s, (size_t)nodes0);
+    sc.prim_min.reserve((size_t)g.final_refs + 1, s, (size_t)ulp0);
+    sc.prim_max.reserve((size_t)g.final_refs + 1, s, (size_t)ulp0);
     ctx->leaf_ids.reserve((size_t)g.nleaf + 1, s, (size_t)nleaf0);
     sc.sub_move.reserve((size_t)moved + 1, s);
     sc.sub_slot[0].reserve((size_t)max_A + 1, s, (size_t)A);

@@ -41,9 +41,11 @@ struct DevBuf {
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
     ~DevBuf() { if (ptr) (void)hipFree(ptr); }
-    // ensure capacity >= n elements; keeps the first `keep` elements
+    // ensure capacity >= n elements; keeps the first `keep` elements (of those
+    // it holds: to keep more than its capacity would read past its end)
     void reserve(size_t n, hipStream_t s, size_t keep = 0) {
         if (n <= cap) return;
+        if (keep > cap) throw Error{PM_ERR_INTERNAL, "a buffer grows with more elements to keep than it holds"};
         size_t ncap = cap ? cap : 256;
         while (ncap < n) ncap += ncap / 2 + 256;
         T *np = nullptr;
