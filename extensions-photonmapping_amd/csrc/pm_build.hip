@@ -3626,7 +3626,7 @@ void capture_batch(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4
     // 2. every buffer at its capacity: nothing may allocate while recording
     BuildScratch &sc = ctx->scratch;
     reserve_build_caps(ctx, caps, N, s);
-    if (ray_order_applies(tp, nrays)) reserve_ray_order(ctx, nrays, s);
+    if (ray_order_used(tp, nrays, caps.leaf_refs)) reserve_ray_order(ctx, nrays, s);   // (the slots it traces with)
     sc.trace_work.reserve(1, s);
     // the batch's own copy of its mesh offsets (eager builds rewrite the scratch copy)
     ctx->graph_off.reserve((size_t)M + 1, s);

@@ -367,16 +367,17 @@ void reserve_scan_tmp(BuildScratch &sc, long long n, hipStream_t s);
 int radix_sort_pairs(unsigned *const keys[2], unsigned *const vals[2], int n, int bits, int *hist, int *offs,
                      bool first_hist_ready, bool iota, BuildScratch &sc, hipStream_t s);
 size_t radix_hist_size(long long n);
-// coherent ray order: whether a trace of nrays rays uses it, its buffers
-// (reserved ahead of a graph capture), and the order itself (device array:
-// the ray indices in the order to trace them, valid until the next call on
-// ctx)
+// coherent ray order: whether a trace of nrays rays asks for it, whether it is
+// used on a tree of that many leaf slots, its buffers (reserved ahead of a graph
+// capture), and the order itself (device array: the ray indices in the order to
+// trace them, valid until the next call on ctx)
 bool ray_order_applies(const pm_trace_params &prm, int nrays);
+bool ray_order_used(const pm_trace_params &prm, int nrays, long long slots);
 void reserve_ray_order(pm_ctx *ctx, int nrays, hipStream_t s);
 const unsigned *ray_order(pm_ctx *ctx, const float4 *org, const float4 *dir, const int *ray_root, int nrays,
                           hipStream_t s);
-// rays up to which the allocation-free trace accepts the coherent order (the
-// order is not used below more rays than that, so it needs no sort buffers)
+// rays up to which the allocation-free trace accepts the coherent order (only
+// more rays are sorted, so it needs no sort buffers)
 constexpr int NOALLOC_MAX_ORDERED_RAYS = PM_NOALLOC_MAX_ORDERED_RAYS;
 // pm_static.hip: the allocation-free trace's work counter (a file-scope device
 // variable) on the calling thread's current device, looked up once per device

@@ -36,7 +36,7 @@ constexpr int TB = 256;                          // threads per block (4 waves)
 constexpr int ITEMS = 16;                        // keys per thread and tile
 constexpr int TILE = TB * ITEMS;                 // keys per sort tile
 constexpr int WAVE_KEYS = TILE / (TB / 64);      // consecutive keys ranked by one wave
-constexpr int ORDER_MIN_RAYS = 1 << 17;          // below this the input order is kept
+constexpr int ORDER_MIN_RAYS = 1 << 17;          // fewer are never reordered
 constexpr int ORDER_BITS = 32;
 
 __device__ __forceinline__ unsigned spread3(unsigned x) {   // 6 bits -> bits 0, 3, ..., 15
@@ -299,6 +299,30 @@ size_t radix_hist_size(long long n) { return 256 * (size_t)sort_tiles(n) + 256; 
 
 bool ray_order_applies(const pm_trace_params &prm, int nrays) {
     return prm.ray_order == PM_RAY_ORDER_COHERENT && nrays >= ORDER_MIN_RAYS;
+}
+
+// Whether a trace that asks for the coherent order is sorted.  The sort takes
+// 75 us for 0.3M rays and 250 for 4M, and a wave of neighbouring rays is as slow
+// as its region; what it saves is fetching the tree, which shows once the tree
+// is past the L2 (leaf records of 48 bytes a slot) and the rays are many.  The
+// rays' kind is the caller's to know, so the lines lie where the kind that gains
+// most, bounces, begins to.  Input / coherent order, us, bounces and random
+// probes off and into soups: 25,000 slots, 1.3M rays 752/881, 1217/1397; 124,000
+// slots, 0.9M 1164/1162, 1905/2059; 1.3M 1534/1490, 2553/2630; 1.8M 2004/1925,
+// 3342/3356; 375,000 slots, 0.6M 1521/1523, 2515/2613; 0.9M 2134/1954, 3603/3585;
+// 1.3M 2884/2528, 4920/4796; 2.5M 5123/4129, 8897/8317; 1.26M slots, 0.6M
+// 2482/2527, 4087/4216; 0.9M 3512/3359, 5914/6062; 1.3M 4834/4478, 8135/8171; 10M
+// slots, 0.6M 4853/4937, 7435/7548; 0.9M 6914/6775, 10832/10768; 1.3M 9450/9092,
+// 14930/14796; large triangles (3.6M slots), 0.6M 768/836, 928/1069; 0.9M
+// 1063/1012, 1194/1318; 1.3M 1359/1245, 1502/1595.  Rays shuffled over 256 meshes
+// (23M slots): 0.9M 810/881, 1.3M 1065/1089, 1.8M 1398/1318, 4M 2750/2287.  Of
+// lines from 0.8M to 1.8M rays, those between 0.92M and 1.18M leave bounces and
+// probes the least behind the better order (0.4% on average, 10% at most); of
+// these the one up to which the allocation-free trace, which has no room for a
+// sort, takes such calls.
+constexpr long long ORDER_PAYS_SLOTS = 1 << 17;
+bool ray_order_used(const pm_trace_params &prm, int nrays, long long slots) {
+    return ray_order_applies(prm, nrays) && nrays > NOALLOC_MAX_ORDERED_RAYS && slots >= ORDER_PAYS_SLOTS;
 }
 
 void reserve_ray_order(pm_ctx *ctx, int nrays, hipStream_t s) {

@@ -1333,22 +1333,6 @@ void dispatch(const TreeDev &T, int algo, const RayBatch &R, int S, pm_hit *out,
     }
 }
 
-// Whether a trace that may use the coherent order does.  The sort takes 75 us
-// for 0.3M rays and 250 for 4M, a wave of neighbouring rays is as slow as its
-// region, and what it saves is fetching the tree: that shows once the tree is
-// past the L2 (leaf records of 48 bytes a slot) and the rays are many.
-// Input / coherent order, us: probe rays in soups of 3,000 / 50,000 /
-// 1,000,000 triangles (3.1M slots): 0.3M rays 149/282, 327/491, 429/533; 1M
-// 408/558, 811/1018, 1063/1146; 2M 714/887, 1459/1704, 1872/1854; 4M 1348/1568,
-// 2720/3085, 3517/3219.  Photons' bounces in the last one: 1.2M 746/804, 2.2M
-// 1222/1039; with 0.35M slots 879/913, with 0.98M 1145/1017.  Rays shuffled over
-// 256 meshes (21M slots): 2M 1513/1390, 7.7M 5017/3697; over 64 (3M slots)
-// 1.9M 1021/962; over 64 (0.9M slots) 0.5M 303/388.
-constexpr int ORDER_PAYS_RAYS = 7 << 18;
-constexpr long long ORDER_PAYS_SLOTS = 1 << 19;
-static_assert(NOALLOC_MAX_ORDERED_RAYS < ORDER_PAYS_RAYS, "the allocation-free trace has no sort buffers");
-bool order_pays(const TreeDev &T, int nrays) { return nrays >= ORDER_PAYS_RAYS && T.num_slots >= ORDER_PAYS_SLOTS; }
-
 template <bool WOOP>
 void dispatch_flags(const TreeDev &T, bool skip, bool count, int algo, const RayBatch &R, int S, pm_hit *out,
                     int4 *cnt, const Launch &L, hipStream_t s) {
@@ -1548,7 +1532,7 @@ void trace_rays(pm_ctx *ctx, int algo, const float4 *org, const float4 *dir, int
     const bool skip = prm.leaf_skipping && ctx->has_boxes;
     const int S = prm.stack_size;
     RayBatch R{org, dir, ray_mesh, nullptr, nrays};
-    if (ray_order_applies(prm, nrays) && order_pays(T, nrays))
+    if (ray_order_used(prm, nrays, T.num_slots))
         R.order = ray_order(ctx, org, dir, ray_mesh, nrays, s);
     query_cus(ctx);
     int *work = ext_work;

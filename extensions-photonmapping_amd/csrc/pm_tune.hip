@@ -115,8 +115,9 @@ void autotune(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2,
     }
     if (first) throw Error{PM_ERR_DEPTH, "no leaf threshold builds this geometry"};
     p.lower_size = best_leaf;
-    // 3. stack depth, ray order and step cap on the chosen tree (the order
-    // only matters from the size at which the tracers apply it)
+    // 3. stack depth, ray order and step cap on the chosen tree (the coherent
+    // order is timed from the size at which it may be asked for, and kept only
+    // where the tracers sort: elsewhere it is the input order timed again)
     build_tree(ctx, P0, P1, P2, n, mesh_offsets, M, p, s);
     int best_stack = 8, best_order = PM_RAY_ORDER_INPUT, best_cap = 0;
     float best_t = 0.0f;
@@ -129,7 +130,8 @@ void autotune(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2,
             for (int cap : kCap) {
                 const float t = time_trace(S, order, cap);
                 ++trials;
-                if (first || t < best_t) {
+                if (first || (t < best_t && (order == PM_RAY_ORDER_INPUT ||
+                                             ray_order_used(q, nrays, ctx->num_prim_indices)))) {
                     best_t = t; best_stack = S; best_order = order; best_cap = cap; first = false;
                 }
             }

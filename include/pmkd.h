@@ -114,14 +114,15 @@ typedef struct {
  *                  call (GeometryList::GetWoopValues, GeometryList.cu:103-117)
  *   ray_order      no reference counterpart: PM_RAY_ORDER_INPUT (default)
  *                  traces the rays in input order; PM_RAY_ORDER_COHERENT
- *                  lets the tree tracers run a trace of >= 131072 rays in
+ *                  lets the tree tracers run a large trace in
  *                  the order of a spatial key (origin cell, direction cell;
  *                  mesh first in a forest) so a wave's rays walk similar
  *                  paths -- for incoherent rays (photons, diffuse bounces,
  *                  random probes); rays that are coherent already (camera
  *                  rays in pixel order) only pay for the sort.  It is done
- *                  where it pays (1,835,008 rays or more, 524,288 leaf slots
- *                  or more).  Each ray's
+ *                  where it can pay (more than 1,048,576 rays on a tree of
+ *                  131,072 leaf slots or more; elsewhere the input order is
+ *                  kept).  Each ray's
  *                  record (and counters) is the same either way and goes to
  *                  the ray's own index; brute force and the canvas keep the
  *                  input order.
@@ -255,8 +256,9 @@ int pm_trace(pm_ctx *ctx, int algo, const float *org, const float *dir, int nray
  * allocates nothing: the work counter is a file-scope device variable of the
  * library (held on every GPU the library runs on until the process ends).
  * Limits: at most
- * PM_NOALLOC_MAX_ORDERED_RAYS rays when the coherent order applies (more:
- * PM_ERR_ARG; use PM_RAY_ORDER_INPUT, which has no limit), MOELLER
+ * PM_NOALLOC_MAX_ORDERED_RAYS rays when the coherent order is asked for, since
+ * larger traces may be sorted and a sort needs memory (more: PM_ERR_ARG; use
+ * PM_RAY_ORDER_INPUT, which has no limit), MOELLER
  * intersection only (WOOP: PM_ERR_UNSUPPORTED).  The tree (pm_build /
  * pm_set_tree) must exist.  Every call on one GPU shares that GPU's counter:
  * calls that overlap on one GPU (two streams, two threads) race. */
