@@ -1077,6 +1077,44 @@ __global__ __launch_bounds__(BRUTE_T) void brute_woop_kernel(const float4 *__res
     }
 }
 
+// A lane per ray through every triangle in index order, the triangles staged
+// through LDS (TB at a time): for few triangles and many rays (see
+// brute_lane_per_ray).
+template <bool COUNT, bool WOOP>
+__global__ __launch_bounds__(TB) void brute_lanes_kernel(const float4 *__restrict__ P0,
+                                                         const float4 *__restrict__ P1,
+                                                         const float4 *__restrict__ P2, int ntris,
+                                                         const float4 *__restrict__ org,
+                                                         const float4 *__restrict__ dir, int n,
+                                                         pm_hit *__restrict__ out, int4 *__restrict__ counters) {
+    __shared__ float4 s0[TB], s1[TB], s2[TB];
+    const int r = blockIdx.x * TB + threadIdx.x;
+    const bool live = r < n;
+    f3 o = {0.0f, 0.0f, 0.0f}, d = {0.0f, 0.0f, 1.0f};
+    if (live) { o = mk3(org[r]); d = mk3(dir[r]); }
+    float th = F_INF, tu = 0.0f, tv = 0.0f;
+    int hit = -1;
+    for (int base = 0; base < ntris; base += TB) {
+        const int k = base + threadIdx.x;
+        __syncthreads();
+        if (k < ntris) { s0[threadIdx.x] = P0[k]; s1[threadIdx.x] = P1[k]; s2[threadIdx.x] = P2[k]; }
+        __syncthreads();
+        const int m = min(TB, ntris - base);
+        if (live) {
+            for (int j = 0; j < m; ++j) {
+                const bool h = WOOP ? woop_test(s0[j], s1[j], s2[j], o, d, th, tu, tv)
+                                    : moller_trumbore(mk3(s0[j]), mk3(s1[j]), mk3(s2[j]), o, d, th, tu, tv);
+                if (h) hit = base + j;
+            }
+        }
+    }
+    if (!live) return;
+    pm_hit res = miss_record();
+    if (th < F_INF && hit != -1) { res.id = hit; res.t = th; res.u = tu; res.v = tv; }
+    out[r] = res;
+    if (COUNT) counters[r] = make_int4(0, 0, ntris, 0);
+}
+
 // ---- trace view
 // n = n_dev ? *n_dev : n_host (a captured build passes its device node count)
 __global__ __launch_bounds__(TB) void pack_nodes_kernel(const int8_t *__restrict__ info,
@@ -1445,20 +1483,49 @@ void query_cus(pm_ctx *ctx);
 // More rays a block mean fewer conversions of the triangles' vectors per pair,
 // fewer rays more blocks: the most that still give every CU a block.  65,536
 // rays x 5,316 triangles: 109 us with 128 rays a block, 134 with 64, 187 with
-// 32 (256 need more registers than four waves a SIMD leave); the kernel it
-// replaced, every ray's exact test against every triangle in 1,024 waves, 1,440.
-// Bound by VALU issue: three instructions per pair and matrix tile row.
+// 32 (256 need more registers than four waves a SIMD leave); a lane per ray
+// through every triangle 1,440.  Bound by VALU issue: three instructions per
+// pair and matrix tile row.
+//
+// A block costs some 6 us before its first pair, so where there are many of
+// them and few triangles the lane-per-ray kernel is the better one.  Its time is
+// 0.27 us a triangle (0.3 Woop) until the device is full and grows with the rays
+// then; the others' grows with the rays at once.  Lane per ray / matrix filter,
+// us: 32,768 rays x 24 triangles 9/10, x 48 16/11; 131,072 x 96 29/35, x 192
+// 55/37; 262,144 x 1 9/50, x 128 51/68, x 256 100/73; 2M x 1 16/390, x 192
+// 410/569, x 384 811/676.  Woop's split kernel (64 rays a block): 262,144 x 32
+// 17/20, x 96 39/36; 1M x 1 12/42, x 192 214/221, x 512 557/557; 131,072 and fewer
+// within 1 us up to 24 triangles, slower with more.  So the limits are 30
+// triangles (Woop 8) per 128 rays of a CU, up to the line from which the filter
+// wins at any number of rays (192; Woop: 384, the two are equal from there).
+bool brute_lane_per_ray(const pm_ctx *ctx, int tris, int n, bool woop) {
+    const long long limit = (long long)(woop ? 8 : 30) * n / (128ll * ctx->num_cus);
+    return tris <= std::min<long long>(limit, woop ? 384 : 192);
+}
+
 template <bool COUNT>
-void brute_rays(pm_ctx *ctx, int tris, const float4 *org, const float4 *dir, int n, pm_hit *out, int4 *counters,
-                hipStream_t s) {
+void brute_rays(pm_ctx *ctx, int tris, bool woop, const float4 *org, const float4 *dir, int n, pm_hit *out,
+                int4 *counters, hipStream_t s) {
     query_cus(ctx);
-    auto launch = [&](auto k, int rays) {
-        k<<<(n + rays - 1) / rays, BRUTE_T, 0, s>>>(ctx->p0, ctx->p1, ctx->p2, tris, org, dir, n, out, counters);
+    const float4 *A = ctx->p0, *B = ctx->p1, *C = ctx->p2;
+    if (woop) {
+        A = woop_tris(ctx, tris, s);
+        B = A + tris;
+        C = B + tris;
+    }
+    auto launch = [&](auto k, int rays, int threads) {
+        k<<<(int)(((long long)n + rays - 1) / rays), threads, 0, s>>>(A, B, C, tris, org, dir, n, out, counters);
     };
+    if (brute_lane_per_ray(ctx, tris, n, woop)) {
+        if (woop) launch(brute_lanes_kernel<COUNT, true>, TB, TB);
+        else launch(brute_lanes_kernel<COUNT, false>, TB, TB);
+        return;
+    }
+    if (woop) return launch(brute_woop_kernel<COUNT>, 64, BRUTE_T);
     const long long per_cu = (long long)n / ctx->num_cus;
-    if (per_cu >= 128) launch(brute_kernel<4, COUNT>, 128);
-    else if (per_cu >= 64) launch(brute_kernel<2, COUNT>, 64);
-    else launch(brute_kernel<1, COUNT>, 32);
+    if (per_cu >= 128) launch(brute_kernel<4, COUNT>, 128, BRUTE_T);
+    else if (per_cu >= 64) launch(brute_kernel<2, COUNT>, 64, BRUTE_T);
+    else launch(brute_kernel<1, COUNT>, 32, BRUTE_T);
 }
 
 void query_cus(pm_ctx *ctx) {
@@ -1510,20 +1577,8 @@ void trace_rays(pm_ctx *ctx, int algo, const float4 *org, const float4 *dir, int
     const bool woop = prm.intersection == PM_INTERSECT_WOOP;
     if (algo == PM_TRACE_BRUTE) {
         const int tris = prm.brute_cap > 0 ? std::min(ctx->ntris, prm.brute_cap) : ctx->ntris;
-        if (woop) {
-            const float4 *W = woop_tris(ctx, tris, s);
-            const int blocks = (nrays + 63) / 64;
-            if (counters)
-                brute_woop_kernel<true><<<blocks, BRUTE_T, 0, s>>>(W, W + tris, W + 2ll * tris, tris, org, dir, nrays,
-                                                                  out, counters);
-            else
-                brute_woop_kernel<false><<<blocks, BRUTE_T, 0, s>>>(W, W + tris, W + 2ll * tris, tris, org, dir,
-                                                                   nrays, out, counters);
-        } else if (counters) {
-            brute_rays<true>(ctx, tris, org, dir, nrays, out, counters, s);
-        } else {
-            brute_rays<false>(ctx, tris, org, dir, nrays, out, counters, s);
-        }
+        if (counters) brute_rays<true>(ctx, tris, woop, org, dir, nrays, out, counters, s);
+        else brute_rays<false>(ctx, tris, woop, org, dir, nrays, out, counters, s);
         PM_LAUNCH_CHECK();
         return;
     }
