@@ -870,7 +870,12 @@ __global__ __launch_bounds__(TB) void trace_coop_kernel(TreeDev T, const float4 
 // V)), of u + v <= 1 and of these vectors is below 2^-18.  E = 0.00122 covers
 // their sum, 0.00119.
 // A ray or triangle whose alpha or beta is not in [2^-40, 2^40] (NaN,
-// infinite, degenerate or out of range) gets the zero vector: always listed.
+// infinite, degenerate or out of range) gets the zero vector: always listed.  So
+// does one whose |d| or em is below 2^-60: squared, a length below about 2^-70
+// is a few multiples of 2^-149, off by up to a third, and products of the exact
+// test that small round by more than a part of their size.  (From 2^-60 on a
+// square is exact to 2^-24, and |d| em >= 2^-120 keeps the exact test's products
+// above what 2^-149 roundings change.)
 //
 constexpr int BRUTE_WAVES = 16;          // waves of a block, each with its share of the triangles
 constexpr int BRUTE_T = 64 * BRUTE_WAVES;
@@ -881,6 +886,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ float norm3(f3 a) { return sqrtf(dot3(a, a)); }
 __device__ __forceinline__ bool brute_scale_ok(float x) { return x >= 0x1p-40f && x <= 0x1p40f; }
+__device__ __forceinline__ bool brute_length_ok(float x) { return x >= 0x1p-60f; }
 __device__ __forceinline__ half4 to_half4(f3 a) {
     half4 h;
     h.x = (_Float16)a.x; h.y = (_Float16)a.y; h.z = (_Float16)a.z; h.w = (_Float16)0.0f;
@@ -944,10 +950,11 @@ __global__ __launch_bounds__(BRUTE_T) void brute_kernel(const float4 *__restrict
         for (int t = 0; t < RT; ++t) {
             const int r = min(r0 + 32 * t + col, n - 1);
             const f3 o = sub3(mk3(org[r]), c), d = mk3(dir[r]);
-            const float alpha = norm3(d) * (S + norm3(o));
+            const float len = norm3(d), alpha = len * (S + norm3(o));
             const f3 x = wpart ? cross3(o, d) : f3{d.x * S, d.y * S, d.z * S};
             const float k = 1.0f / alpha;
-            rays[t] = to_half4(brute_scale_ok(alpha) ? f3{x.x * k, x.y * k, x.z * k} : f3{0.0f, 0.0f, 0.0f});
+            const bool ok = brute_scale_ok(alpha) && brute_length_ok(len);
+            rays[t] = to_half4(ok ? f3{x.x * k, x.y * k, x.z * k} : f3{0.0f, 0.0f, 0.0f});
         }
         int pending = 0;
         // tests the list's first m pairs exactly
@@ -975,7 +982,7 @@ __global__ __launch_bounds__(BRUTE_T) void brute_kernel(const float4 *__restrict
                 const f3 v0 = sub3(p0, c), e1 = sub3(p1, p0), e2 = sub3(p2, p0);
                 const float em = norm3(e1) + norm3(e2);
                 const float beta = em * (S + norm3(v0) + em) / S;
-                const bool ok = brute_scale_ok(beta);
+                const bool ok = brute_scale_ok(beta) && brute_length_ok(em);
                 f3 g1, g2, g3;
                 float k = 1.0f / beta;
                 if (wpart) {
