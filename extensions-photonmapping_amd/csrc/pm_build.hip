@@ -3193,14 +3193,18 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
     // take longer, 650 -> 637).  The build ends after the level that creates no active node; a
     // level launched past it has no nodes and writes none.
     LevelSizes known{M, N, S_now, M, 0, 0};   // the level after the last one whose state is known
-    int known_max = 0;                        // the largest node of the known level
+    int known_max = ctx->largest_mesh;        // the largest node of the known level (INT_MAX: not looked at)
     // the subtrees of a small build's level whose nodes hold up to SUB_MAX refs (a captured
     // batch keeps its buffers, and the DIVIDE split its own passes; with small
-    // leaves the straddling refs outgrow a subtree's room)
+    // leaves the straddling refs outgrow a subtree's room).  Not where the largest
+    // node has one level to go: the subtrees are four launches and a wait, a level
+    // three.  Nor on a level of more nodes than its refs fill: a forest's roots may
+    // be any number, and each takes a block and 32 records.
     bool subtrees = run_ahead && !div && LS >= 16 && N <= SUB_REFS;
-    auto to_subtrees = [&]() { return subtrees && known_max <= SUB_MAX && known.R <= 2 * SUB_REFS; };
-    for (int m = 0; subtrees && m < M; ++m)
-        known_max = std::max(known_max, ctx->mesh_offsets[m + 1] - ctx->mesh_offsets[m]);
+    auto to_subtrees = [&]() {
+        return subtrees && known_max <= SUB_MAX && known_max >= 2 * LS && known.R <= 2 * SUB_REFS &&
+               known.A * LS <= known.R;
+    };
     std::deque<unsigned> out;                 // levels launched after that, not taken yet
     bool done = false;
     for (int lvl = 0; graph ? lvl < caps->upper_levels : !done; ++lvl) {
@@ -3257,8 +3261,10 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
         PM_LAUNCH_CHECK();
         if (graph) continue;
         out.push_back(seq);
-        auto ahead = [&]() {   // (a level whose nodes go to subtrees is not launched)
-            return run_ahead && known.R <= AHEAD_REFS && !to_subtrees() ? 1u : 0u;
+        // (a level whose nodes go to subtrees is not launched, nor one after roots
+        // that hold no node's refs)
+        auto ahead = [&]() {
+            return run_ahead && known.R <= AHEAD_REFS && known_max >= LS && !to_subtrees() ? 1u : 0u;
         };
         while (!done && out.size() > ahead()) {
             const int taken = (lvl + 1 - (int)out.size()) & 1;   // the taken level's parity
@@ -3276,7 +3282,7 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
             Lvl n = h;
             advance_level(&n);
             known = LevelSizes{n.A, n.R, h.scanS[taken ^ 1], n.nodes_size, n.final_refs, n.nleaf};
-            known_max = (int)h.max_child;
+            known_max = subtrees ? (int)h.max_child : INT_MAX;
         }
     }
     // the last level's advance
@@ -3413,9 +3419,15 @@ void upload_offsets(pm_ctx *ctx, const int *mesh_offsets, int N, int M, hipStrea
         off_h[0] = 0;
         off_h[1] = N;
     }
-    for (int m = 0; m < M; ++m)
-        if (off_h[m] > off_h[m + 1]) throw Error{PM_ERR_ARG, "mesh offsets must be non-decreasing"};
+    int smallest = 0, largest = 0;
+    for (int m = 0; m < M; ++m) {
+        const int size = (int)((unsigned)off_h[m + 1] - (unsigned)off_h[m]);
+        smallest = std::min(smallest, off_h[m] > off_h[m + 1] ? -1 : 0);
+        largest = std::max(largest, size);
+    }
+    if (smallest < 0) throw Error{PM_ERR_ARG, "mesh offsets must be non-decreasing"};
     if (off_h[0] != 0 || off_h[M] != N) throw Error{PM_ERR_ARG, "mesh offsets must span [0, n]"};
+    ctx->largest_mesh = largest;
     sc.mesh_off.reserve((size_t)M + 1, s);
     if (M > 1) {   // (a single mesh's {0, N} is never read: no copy and no stream wait)
         PM_HIP(hipMemcpyAsync(sc.mesh_off.ptr, off_h.data(), (M + 1) * sizeof(int), hipMemcpyHostToDevice, s));

@@ -269,6 +269,7 @@ struct pm_ctx {
     std::vector<long long> level_refs;
     int num_roots = 1;                 // meshes in the last build (roots 0..num_roots-1)
     std::vector<int> mesh_offsets;     // triangle offsets per mesh (host copy)
+    int largest_mesh = 0;              // triangles of the largest (of the last build's)
     pmkd::BuildSizes last_sizes;       // what the last eager build reached
     long long last_ntris = -1;         // its triangle count (-1: no build yet)
     bool planned_build = false;        // the last build ran with capacities from the one before it
