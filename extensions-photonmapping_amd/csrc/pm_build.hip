@@ -514,7 +514,9 @@ constexpr int NT = NPT * LBS;          // active nodes per tile
 // A status word is flag << 62 | value: flag 1 = aggregate, 2 = inclusive prefix.
 constexpr unsigned long long LB_AGG = 1ull << 62, LB_INC = 2ull << 62, LB_VAL = LB_AGG - 1;
 // A wait for a predecessor is bounded: a tile that never publishes (only
-// possible through a bug) fails the build instead of hanging it.
+// possible through a bug) fails the build instead of hanging it.  The tile that
+// gives up sets the status and publishes no prefix, so that no later tile takes
+// a wrong one for its own.
 constexpr int LB_SPIN = 1 << 22;
 
 __device__ __forceinline__ unsigned long long lb_load(const unsigned long long *w) {
@@ -528,10 +530,11 @@ __device__ __forceinline__ void lb_store(unsigned long long *w, unsigned long lo
 // aggregates are agg[k]; the status word of (tile, k) is w[K * tile + k].
 // The K look-backs run side by side: lanes 8k .. 8k+7 walk count k's words
 // over windows of 8 predecessors (lane 8k + j reads tile base - j), each
-// group stopping at its nearest inclusive prefix.
+// group stopping at its nearest inclusive prefix.  false (and excl not the
+// prefixes): gave up after `limit` waits.
 template <int K>
-__device__ void lookback(unsigned long long *__restrict__ w, int tile, const long long *agg, long long *excl,
-                         int *status) {
+__device__ bool lookback(unsigned long long *__restrict__ w, int tile, const long long *agg, long long *excl,
+                         int *status, int limit = LB_SPIN) {
     static_assert(K >= 1 && K <= 8, "one group of 8 lanes per count");
     const int lane = __lane_id();
     const int k = lane >> 3, j = lane & 7;
@@ -542,13 +545,19 @@ __device__ void lookback(unsigned long long *__restrict__ w, int tile, const lon
         if (j == 0 && k < K) lb_store(&w[k], LB_INC | (unsigned long long)a);
 #pragma unroll
         for (int q = 0; q < K; ++q) excl[q] = 0;
-        return;
+        return true;
     }
     if (j == 0 && k < K) lb_store(&w[(long long)K * tile + k], LB_AGG | (unsigned long long)a);
     long long sum = 0;                     // the group's predecessors summed so far (same in its 8 lanes)
     bool done = k >= K;
     int base = tile - 1, spins = 0;
+    bool gave_up = false;
     while (__ballot(!done)) {
+        if (spins > limit) {
+            if (lane == 0) atomicCAS(status, 0, PM_ERR_INTERNAL);
+            gave_up = true;
+            break;
+        }
         unsigned long long v = LB_INC;
         if (!done) {
             const int idx = base - j;
@@ -570,16 +579,14 @@ __device__ void lookback(unsigned long long *__restrict__ w, int tile, const lon
             else base -= 8;
         }
         if (__ballot(!done && !ready)) {                   // a predecessor has not published yet
-            if (++spins > LB_SPIN) {
-                if (lane == 0) atomicCAS(status, 0, PM_ERR_INTERNAL);
-                break;
-            }
+            ++spins;
             __builtin_amdgcn_s_sleep(2);
         }
     }
 #pragma unroll
     for (int q = 0; q < K; ++q) excl[q] = __shfl(sum, 8 * q, 64);
-    if (j == 0 && k < K) lb_store(&w[(long long)K * tile + k], LB_INC | (unsigned long long)(sum + a));
+    if (j == 0 && k < K && !gave_up) lb_store(&w[(long long)K * tile + k], LB_INC | (unsigned long long)(sum + a));
+    return !gave_up;
 }
 
 // the block's next tile (ticket order); every thread returns the same value.
@@ -1800,6 +1807,7 @@ __global__ __launch_bounds__(SUB_WORDS) void sub_publish_kernel(int *__restrict_
 struct NumArgs {
     int A, active_index, child_start, next_active, leaf_nodes, leaf_left, L_all, LL_all, ulp, nleaf, nleaf0;
     int LS, propagate, par, depth;
+    int spins;                         // waits after which a look-back gives up
     const int4 *rec;
     const int *slot;
     int *slot_n;
@@ -1810,17 +1818,21 @@ struct NumArgs {
 
 // The nodes of a level, one per thread: the scans, chains and child records
 // the leaf and scatter passes make.  Everything of the level is written in this
-// one launch, since the totals that number the right children are known.
+// one launch, since the totals that number the right children are known.  A tile
+// whose look-back gave up writes nothing, and the levels after it (whose slots
+// it would have written) do not start.
 __global__ __launch_bounds__(LBS) void number_pass_kernel(NodePtrs N, Lvl *L, NumArgs P,
                                                          int *__restrict__ leaf_ids) {
-    __shared__ int s_tile;
+    __shared__ int s_tile, s_ok;
     __shared__ int s_w[7][LBS / 64];
     __shared__ long long s_ex[7];
     const int t = threadIdx.x;
     if (t == 0) {
+        s_ok = L->status == 0;
         s_tile = atomicAdd(&P.ctr[P.par], 1);
     }
     __syncthreads();
+    if (!s_ok) return;
     const int tile = s_tile;           // (as many blocks as tiles)
     const int i = tile * LBS + t, node = P.active_index + i;
     const bool in_tile = i < P.A;
@@ -1842,11 +1854,14 @@ __global__ __launch_bounds__(LBS) void number_pass_kernel(NodePtrs N, Lvl *L, Nu
     if (t < 64) {
         const long long agg[7] = {tot[0], tot[1], tot[2], tot[3], tot[4], tot[5], tot[6]};
         long long ex[7];
-        lookback<7>(P.lb, tile, agg, ex, &L->status);
-        if (t == 0)
+        const bool ok = lookback<7>(P.lb, tile, agg, ex, &L->status, P.spins);
+        if (t == 0) {
+            s_ok = ok;
             for (int k = 0; k < 7; ++k) s_ex[k] = ex[k];
+        }
     }
     __syncthreads();
+    if (!s_ok) return;
     if (in_tile) {
         const f3 rMin = {__int_as_float(r0.x), __int_as_float(r0.y), __int_as_float(r0.z)};
         const f3 rMax = {__int_as_float(r1.x), __int_as_float(r1.y), __int_as_float(r1.z)};
@@ -1904,16 +1919,23 @@ __global__ __launch_bounds__(LBS) void number_pass_kernel(NodePtrs N, Lvl *L, Nu
 }
 
 // The subtrees' leaf refs to their places, 16 lanes a leaf; the level state
-// after the last level.
+// after the last level, and its status to the host (nothing after the subtrees
+// need read the state back).  Where a look-back gave up some leaves' entries were
+// not written: none is moved.
 constexpr int MOVE_LANES = 16;
 __global__ __launch_bounds__(BS) void leaf_move_kernel(Lvl *L, Lvl v, const int4 *__restrict__ mv, int n,
                                                        const float4 *__restrict__ xmin,
                                                        const float4 *__restrict__ xmax, float4 *__restrict__ fmin,
-                                                       float4 *__restrict__ fmax) {
+                                                       float4 *__restrict__ fmax, unsigned long long *host,
+                                                       unsigned seq) {
+    const int status = L->status;   // (what is stored below leaves it as it is)
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        if (L->status) lvl_fail(&v, L->status);   // a look-back that failed
+        if (status) lvl_fail(&v, status);
         *L = v;
+        __hip_atomic_store(host, (unsigned long long)seq << 32 | (unsigned)status, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
     }
+    if (status) return;
     const int lane = threadIdx.x % MOVE_LANES;
     for (int k = (blockIdx.x * BS + threadIdx.x) / MOVE_LANES; k < n; k += gridDim.x * BS / MOVE_LANES) {
         const int4 m = mv[k];
@@ -2962,9 +2984,10 @@ void reserve_first(pm_ctx *ctx, int N, int M, int seg, hipStream_t s) {
 // subtree_kernel).  h: the level state with that level's advance to come; on
 // success the state after the last level (on the device too).  false, and
 // nothing changed, when the subtrees cannot hold the build: the level loop
-// goes on and reports what there is to report.
+// goes on and reports what there is to report.  moved_seq: the number of the record
+// (the first word of the subtrees') that gives the status of the passes launched.
 bool build_subtrees(pm_ctx *ctx, Lvl &h, int par, int S, int max_n, const pm_build_params &prm, int seg,
-                    BuildSizes &seen, hipStream_t s) {
+                    BuildSizes &seen, unsigned &moved_seq, hipStream_t s) {
     BuildScratch &sc = ctx->scratch;
     const int nxt = par ^ 1, LS = prm.lower_size;
     Lvl g = h;
@@ -3059,7 +3082,11 @@ bool build_subtrees(pm_ctx *ctx, Lvl &h, int par, int S, int max_n, const pm_bui
     sc.lb_words[par].reserve((size_t)words, s, 8 * (size_t)((A + LBS - 1) / LBS));
     sc.lb_words[nxt].reserve((size_t)words, s);
     const NodePtrs NP = node_ptrs(ctx);
+    // (a test makes every look-back over more than one tile give up at once)
+    const char *const limit = std::getenv("PMKD_LOOKBACK_SPINS");
+    const int spins = limit ? std::atoi(limit) : LB_SPIN;
     for (NumArgs &P : plans) {
+        P.spins = spins;
         P.rec = sc.sub_rec.ptr;
         P.slot = sc.sub_slot[P.depth & 1].ptr;
         P.slot_n = sc.sub_slot[(P.depth & 1) ^ 1].ptr;
@@ -3070,8 +3097,8 @@ bool build_subtrees(pm_ctx *ctx, Lvl &h, int par, int S, int max_n, const pm_bui
         PM_LAUNCH_CHECK();
     }
     leaf_move_kernel<<<grid_for((long long)moved * MOVE_LANES, BS, 1 << 16), BS, 0, s>>>(
-        sc.lvl.ptr, g, sc.sub_move.ptr, moved, a.xmin, a.xmax, sc.prim_min.ptr,
-        sc.prim_max.ptr);
+        sc.lvl.ptr, g, sc.sub_move.ptr, moved, a.xmin, a.xmax, sc.prim_min.ptr, sc.prim_max.ptr, sc.mirror.sub_dev,
+        moved_seq = sc.mirror.take_seq());
     PM_LAUNCH_CHECK();
     ctx->level_refs.insert(ctx->level_refs.end(), level_refs.begin(), level_refs.end());
     seen = sn;
@@ -3205,12 +3232,13 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
         return subtrees && known_max <= SUB_MAX && known_max >= 2 * LS && known.R <= 2 * SUB_REFS &&
                known.A * LS <= known.R;
     };
+    unsigned moved_seq = 0;                   // the subtrees' final status, to be taken (0: no subtrees)
     std::deque<unsigned> out;                 // levels launched after that, not taken yet
     bool done = false;
     for (int lvl = 0; graph ? lvl < caps->upper_levels : !done; ++lvl) {
         const int par = lvl & 1, nxt = par ^ 1;
         if (out.empty() && to_subtrees()) {
-            if (build_subtrees(ctx, h, par, (int)known.S, known_max, prm, seg, seen, s)) break;
+            if (build_subtrees(ctx, h, par, (int)known.S, known_max, prm, seg, seen, moved_seq, s)) break;
             subtrees = false;
         }
         LevelSizes b = known;
@@ -3408,6 +3436,10 @@ void run_build(pm_ctx *ctx, const float4 *P0, const float4 *P1, const float4 *P2
         ctx->num_nodes = (int)caps->nodes;
     }
     build_node_view(ctx, s, graph ? &L->nodes_size : nullptr);
+    if (moved_seq) {   // (the launches since are on their way)
+        wait_words(sc.mirror.sub_host, &h.status, 1, moved_seq, s);
+        if (h.status) throw_status(h);
+    }
 }
 
 void upload_offsets(pm_ctx *ctx, const int *mesh_offsets, int N, int M, hipStream_t s) {
