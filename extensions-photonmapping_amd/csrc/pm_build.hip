@@ -2962,22 +2962,48 @@ struct LevelSizes {
 // context's first build does not grow them level by level: every growth is an
 // allocation, a copy and a wait (a context's first build of 1,000,002
 // triangles 11.1 -> 2.7 ms, of 256 meshes with 10.3M 28.9 -> 14.3 ms).  Larger
-// needs still grow.
+// needs still grow.  It is a guess, so it takes at most half of the free memory
+// (the buffers that come after take less than these), and where it cannot be
+// had the levels size their buffers as they go.
 void reserve_first(pm_ctx *ctx, int N, int M, int seg, hipStream_t s) {
     BuildScratch &sc = ctx->scratch;
     const long long n = N, r = (n <= AHEAD_REFS ? 8 : 5) * n, a = n / 8 + 2ll * M;
-    for (int q = 0; q < 2; ++q) {
-        sc.ref_min[q].reserve((size_t)r + 1, s);
-        sc.ref_max[q].reserve((size_t)r + 1, s);
-        sc.keys[q].reserve((size_t)std::max(12 * a, key_words_host(2 * JOIN_TEST_NODES, true)) + 6, s);
-        sc.node_segbase[q].reserve((size_t)(2 * a) + 2, s);
-        sc.segs[q].reserve((size_t)(2 * a + r / seg) + 1, s);
+    const long long keys = std::max(12 * a, key_words_host(2 * JOIN_TEST_NODES, true)) + 6;
+    const long long nodes = n + n / 2 + 1024 + 16ll * M;
+    // (a buffer's capacity is up to half more than asked for)
+    const size_t bytes = 3 * ((size_t)r * 6 * sizeof(float4) + (size_t)keys * 2 * sizeof(int) +
+                              (size_t)(2 * a + r / seg) * (2 * sizeof(int4) + 4 * sizeof(int)) +
+                              (size_t)a * (3 * sizeof(int4) + 4 * sizeof(int)) + (size_t)nodes * 65 +
+                              (size_t)(n / 2 + 2 * M) * sizeof(int)) / 2;
+    size_t free_bytes = 0, all = 0;
+    if (hipMemGetInfo(&free_bytes, &all) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
     }
-    for (DevBuf<int> *b : {&sc.segL, &sc.segR, &sc.segLoff, &sc.segRoff}) b->reserve((size_t)(a + r / seg) + 1, s);
-    sc.node_rec.reserve(3 * (size_t)a + 3, s);
-    sc.prim_min.reserve((size_t)r + 1, s); sc.prim_max.reserve((size_t)r + 1, s);
-    ctx->leaf_ids.reserve((size_t)n / 2 + 2 * M, s);
-    ctx->nodes.reserve((size_t)(n + n / 2) + 1024 + 16 * M, s, 0);
+    if (bytes > free_bytes / 2) return;
+    try {
+        for (int q = 0; q < 2; ++q) {
+            sc.ref_min[q].reserve((size_t)r + 1, s);
+            sc.ref_max[q].reserve((size_t)r + 1, s);
+            sc.keys[q].reserve((size_t)keys, s);
+            sc.node_segbase[q].reserve((size_t)(2 * a) + 2, s);
+            sc.segs[q].reserve((size_t)(2 * a + r / seg) + 1, s);
+        }
+        for (DevBuf<int> *b : {&sc.segL, &sc.segR, &sc.segLoff, &sc.segRoff}) b->reserve((size_t)(a + r / seg) + 1, s);
+        sc.node_rec.reserve(3 * (size_t)a + 3, s);
+        sc.prim_min.reserve((size_t)r + 1, s); sc.prim_max.reserve((size_t)r + 1, s);
+        ctx->leaf_ids.reserve((size_t)n / 2 + 2 * M, s);
+        ctx->nodes.reserve((size_t)nodes, s, 0);
+    } catch (const Error &) {
+        (void)hipGetLastError();
+        for (int q = 0; q < 2; ++q) {
+            sc.ref_min[q].release(); sc.ref_max[q].release();
+            sc.keys[q].release(); sc.node_segbase[q].release(); sc.segs[q].release();
+        }
+        for (DevBuf<int> *b : {&sc.segL, &sc.segR, &sc.segLoff, &sc.segRoff}) b->release();
+        sc.node_rec.release(); sc.prim_min.release(); sc.prim_max.release();
+        ctx->leaf_ids.release();
+    }
 }
 
 // The upper stage's remaining levels by the subtrees of level `par`'s nodes (see

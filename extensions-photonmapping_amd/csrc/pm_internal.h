@@ -40,7 +40,12 @@ struct DevBuf {
     DevBuf() = default;
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
-    ~DevBuf() { if (ptr) (void)hipFree(ptr); }
+    ~DevBuf() { release(); }
+    void release() {
+        if (ptr) (void)hipFree(ptr);
+        ptr = nullptr;
+        cap = 0;
+    }
     // ensure capacity >= n elements; keeps the first `keep` elements (of those
     // it holds: to keep more than its capacity would read past its end)
     void reserve(size_t n, hipStream_t s, size_t keep = 0) {
