@@ -1484,8 +1484,10 @@ __host__ __device__ void advance_level(Lvl *L) {
 // many waves as a depth has nodes: 16 and 8 (8 and 4 measured 2% slower on
 // builds of 5,000 to 100,000 triangles).  Where a level fills the device it is
 // instruction issue that counts, about 800 instructions a node against the
-// level passes' streaming: 1,000,002 triangles 1.41 ms without subtrees and
-// 1.54 ms with them, hence SUB_REFS.
+// level passes' streaming: 1,000,002 clustered triangles 1.41 ms without
+// subtrees and 1.54 ms with them.  SUB_REFS is a line well inside the sizes where
+// they gain: builds of uniform soups of 131,072 triangles 457 us without and 354
+// with them, of 200,000 497 and 400, of 500,000 611 and 529.
 // Rebuilds, before and after: a 5,316-triangle room 702 -> 570 us, soups of
 // 2,000 / 10,000 / 100,000 triangles 328 / 446 / 650 -> 260 / 350 / 603 us, a
 // 31,752-triangle terrain 430 -> 350 us.
@@ -2499,7 +2501,9 @@ __global__ __launch_bounds__(WPB * 64) void sah_kernel(
 // A 5,316-triangle room with 8 lower levels of up to 2,334 nodes 574 -> 536 us.
 // Without forced splits the screen settles most nodes lane by lane, and a wave
 // for each costs more (soups of 2,000 triangles 262 -> 281 us); larger levels
-// keep their waves for the nodes that need the search.
+// keep their waves for the nodes that need the search.  Whole builds with forced
+// splits, apart / in one launch: 4,007 upper leaves 519 / 496 us, 6,333 560 / 598,
+// 11,199 697 / 821.
 constexpr int LOWER_SMALL = 4096;
 __global__ __launch_bounds__(WPB * 64) void sah_level_kernel(
     NodePtrs N, const int *__restrict__ leaf_ids, const Lvl *__restrict__ L, const float4 *__restrict__ pmin,
@@ -2619,6 +2623,8 @@ __device__ void plan_lower_apply(Lvl *L, int splits, unsigned long long c) {
 // eager build (mirror) also publishes the state.
 // Scan, plan and advance as launches of their own were 8 us a level and the
 // gaps between them; a level of more nodes is scanned by more than one block.
+// Whole builds, scanned before / here: 6,333 upper leaves 557 / 560 us, 11,199 706 /
+// 697, 16,809 751 / 770, 29,742 901 / 960.
 constexpr int PLAN_T = 1024, PLAN_SCAN = 4 * 4 * PLAN_T;
 template <bool SCAN>
 __global__ __launch_bounds__(PLAN_T) void plan_lower_kernel(Lvl *L, const int *__restrict__ flag,
@@ -2941,9 +2947,14 @@ inline int grid_for(long long n, int per, int cap) {
 
 // refs of a level up to which an eager build launches one level ahead of the
 // state it has taken (the ahead level's buffers are reserved for twice its
-// bound)
+// bound).  Where many levels come before the subtrees it pays (a 5,144-triangle
+// room 383 -> 345 us); where few do, the level launched ahead can be one that the
+// subtrees would have taken (soups of 8,000 and 70,000 triangles 217 -> 245, 319 ->
+// 347).  Levels of more refs: no difference (200,000 triangles 505 / 497, 500,000
+// 605 / 612).  The lower levels' line: builds with forced splits, without / with,
+// 112 upper leaves 281 / 240 us, 1,104 382 / 364, 6,333 576 / 560, 16,809 751 / 745.
 constexpr long long AHEAD_REFS = 1 << 17;
-constexpr long long AHEAD_NODES = 1 << 14;   // the same for the nodes of a lower level
+constexpr long long AHEAD_NODES = 1 << 14;   // nodes of a lower level, likewise
 constexpr long long SUB_REFS = 1 << 17;      // triangles of a build up to which its nodes go to subtrees (subtree_kernel),
                                              // while a level has at most twice as many refs
 
