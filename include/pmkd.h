@@ -246,7 +246,10 @@ int pm_tree_stats(pm_ctx *ctx, pm_stats *out, void *stream);
  * BruteTracer.cu:123-172) with the ray arrays passed in (float4 org/dir per
  * ray, device) and the first hit of each ray written to out (device) instead
  * of a shaded canvas.  counters (device int[4*nrays] or NULL): per ray
- * inner-node visits, leaf visits, triangle tests, leaf-box tests. */
+ * inner-node visits, leaf visits, triangle tests, leaf-box tests.  KD_RESTART's
+ * inner-node counter counts every restart from the root; without counters the
+ * call resumes where it can instead (same records, leaves and triangle tests,
+ * fewer inner nodes), so a counted call also takes longer. */
 int pm_trace(pm_ctx *ctx, int algo, const float *org, const float *dir, int nrays,
              pm_hit *out, const pm_trace_params *params, int *counters, void *stream);
 
